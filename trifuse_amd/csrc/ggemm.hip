@@ -40,6 +40,18 @@
 #include "tfm_device.h"
 #include "tfm_internal.h"
 
+// Compiled once per storage dtype and code width, so that the instances build
+// in parallel: as is for 4-bit codes with bf16 storage (which also holds the
+// launch functions), and from ggemm_f16.hip, ggemm_i8.hip and
+// ggemm_f16_i8.hip for the others.
+#ifndef TFM_GG_F16
+#define TFM_GG_F16 0
+#endif
+#ifndef TFM_GG_BITS
+#define TFM_GG_BITS 4
+#endif
+#define TFM_GG_MAIN (TFM_GG_BITS == 4 && !TFM_GG_F16)
+
 namespace tfm {
 
 constexpr int BK = 64;
@@ -56,11 +68,7 @@ struct GgArgs {
   int N;                 // output columns of one matrix
   int Kin;
   uint16_t* out;         // gate/up: h [n_routes, N]; down: y [n_routes, N]; plain: out [rows, N]
-  int sb_layout;         // ggemm_wr_kernel's scale/bias layout in LDS (kSbPlain, kSbDword, kSbChunk)
 };
-
-// Scale/bias layouts of ggemm_wr_kernel's LDS copy (see there).
-enum { kSbPlain = 0, kSbDword = 1, kSbChunk = 2 };
 
 // Row of accumulator element v of lane `lane` inside a 32x32 block of
 // v_mfma_f32_32x32x16_bf16 (its column is lane % 32; operands: lane l
@@ -521,12 +529,9 @@ __global__ __launch_bounds__(WAVES_M_ * WAVES_N_ * 64, 1) void ggemm_kernel(GgAr
   });
 }
 
-// Tile shapes (eight waves each): 256 x 256 (2 x 4 waves of 128 x 64) when
-// the experts hold enough routes to fill 256-row tiles, 128 x 256 (2 x 4
-// waves of 64 x 64) otherwise. TFM_GGEMM_TILE=256 or 128 forces one of them.
 // ---------------------------------------------------------------------------
-// 4-bit weights with inputs up to 2048 wide, a multiple of 128: the weights
-// stay in registers.
+// 4- and 8-bit weights with inputs a multiple of 128 wide: the weights stay
+// in registers.
 //
 // Tile: BM routed rows x 256 weight rows, eight waves. Wave w owns 32 weight
 // rows (gate/up: gate rows 16w..16w+15 and the same up rows; down and plain:
@@ -537,21 +542,22 @@ __global__ __launch_bounds__(WAVES_M_ * WAVES_N_ * 64, 1) void ggemm_kernel(GgAr
 //
 // Per super-step of 128 k (two quantisation groups):
 //   * the BM activation rows are copied into LDS (one of two stages);
-//   * lane l loads 16 contiguous bytes (32 codes) of each of its two weight
-//     rows: k = 32 (l / 16) .. + 31 of the super-step, which share one scale
-//     group. Word s of them (k = 32 (l / 16) + 8 s .. + 7) is dequantised
-//     into the B operand of sub-step s. The reduction order inside an MFMA is
-//     free, so the A operand of sub-step s for lane l is the same k range:
-//     LDS chunk 4 (l / 16) + s of the row;
+//   * lane l loads the 32 contiguous codes (16 or 32 bytes) k = 32 (l / 16)
+//     .. + 31 of the super-step of each of its two weight rows; they share one
+//     scale group. Codes 8 s .. 8 s + 7 of them are dequantised into the B
+//     operand of sub-step s. The reduction order inside an MFMA is free, so
+//     the A operand of sub-step s for lane l is the same k range: LDS chunk
+//     4 (l / 16) + s of the row;
 //   * one barrier, for the next stage's activations.
 // Every packed weight is dequantised exactly once per tile and never goes
-// through LDS; scales and biases of the tile's rows are copied into LDS once
-// per tile. Per 128 k a wave runs 4 x BM/8 MFMAs for one barrier, twice the
+// through LDS. Per 128 k a wave runs 4 x BM/8 MFMAs for one barrier, twice the
 // work per barrier of the kernel above.
 //
 // LDS: activation row r of a stage is 256 B (16 chunks of 16 B); chunk c is
 // stored in slot c ^ (r & 15), so the 16 lanes of one read pass (16
-// consecutive rows, one chunk) hit distinct bank groups.
+// consecutive rows, one chunk) hit distinct bank groups. The scales and
+// biases of the tile's rows are kept for four super-steps at a time (eight
+// groups, 16 bytes a row) in a ring of two.
 constexpr int BK2 = 128;
 
 __device__ __forceinline__ f32x4_t mfma16(bf16x8_t a, bf16x8_t b, f32x4_t c, std::false_type) {
@@ -561,21 +567,102 @@ __device__ __forceinline__ f32x4_t mfma16(f16x8_t a, f16x8_t b, f32x4_t c, std::
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
 
-// BM = 64 (few routes per expert): 64 KB of LDS and 32 accumulator
-// registers, so two workgroups share a compute unit and each covers the
-// other's weight-load latency, which a super-step's few MFMAs cannot. WV = 4
-// (64-row tiles only) halves the weight rows of a tile (128: 64 gate and 64
-// up rows, or 128 down rows) for twice the tiles, where 8-wave tiles would
-// leave compute units idle (a few experts or a few output columns: Granite
-// decode batches, a dense matrix); 48 KB of LDS, three workgroups per
-// compute unit.
-template <int BM, int MODE, bool F16, int WV, bool FEW = false>
-__global__ __launch_bounds__(WV * 64, BM == 64 ? (WV == 8 ? 2 : 3) : 1) void ggemm_wr_kernel(GgArgs args) {
+// Dequantisation of 8 codes (one lane's share of a sub-step) into four packed
+// pairs, cut into eight slices 0..7 that the main loop spreads over its MFMAs.
+// Scale and bias as loaded once per super-step: floats for bf16, (s, s) pairs
+// for half.
+//
+// 4-bit: a byte 0..15 read as fp8 (e4m3, subnormal below 8) is code / 512, so
+// one v_cvt_scalef32_pk with scale 512 turns two codes into two exact floats
+// (v_cvt_f32_ubyte turns one, at the same cost: 5 cycles per wave
+// instruction). bf16 then takes fp32 fused multiply-adds and one rounding.
+// Half multiplies and adds in half: v_pk_fma_f16 rounds the exact s q + b once
+// (codes and 11-bit scales are exact in half), where fp32 followed by a
+// conversion rounds twice.
+// 8-bit: bf16 converts byte by byte; half takes 1024 + q (the byte under an
+// exponent byte) minus 1024, both exact, then the same fused multiply-add.
+template <int BITS, bool F16>
+struct Deq8 {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+  using sb_t = std::conditional_t<F16, f16x2, float>;
+  static constexpr int WORDS = BITS / 4;          // packed words of 8 codes
+
+  uint32_t lo, hi;
+  f32x2 pl, ph;
+  f16x2 p16;
+  float f;
+
+  static __device__ __forceinline__ sb_t sb(uint16_t h) {
+    if constexpr (F16) {
+      const _Float16 v = __builtin_bit_cast(_Float16, h);
+      return f16x2{v, v};
+    } else {
+      return bf2f(h);
+    }
+  }
+
+  // out: the four packed pairs; w: the WORDS packed words.
+  template <int EL>
+  __device__ __forceinline__ void slice(const uint32_t* w, sb_t s, sb_t b, uint32_t* out) {
+    constexpr int half = EL / 4, e4 = EL % 4;
+    if constexpr (BITS == 4 && !F16) {
+      if constexpr (EL == 0) {
+        lo = w[0] & 0x0f0f0f0fu;                  // codes 0 2 4 6
+        hi = (w[0] >> 4) & 0x0f0f0f0fu;           // codes 1 3 5 7
+      }
+      if constexpr (e4 == 0) pl = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(lo, 512.0f, half == 1);
+      if constexpr (e4 == 1) ph = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(hi, 512.0f, half == 1);
+      if constexpr (e4 == 2)
+        out[2 * half] = pack_bf16x2(__builtin_fmaf(s, pl[0], b), __builtin_fmaf(s, ph[0], b));
+      if constexpr (e4 == 3)
+        out[2 * half + 1] = pack_bf16x2(__builtin_fmaf(s, pl[1], b), __builtin_fmaf(s, ph[1], b));
+    } else if constexpr (BITS == 4) {
+      if constexpr (EL == 0) {
+        lo = w[0] & 0x0f0f0f0fu;
+        hi = (w[0] >> 4) & 0x0f0f0f0fu;
+      }
+      if constexpr (EL == 1) {
+        const uint32_t l = lo;
+        lo = __builtin_amdgcn_perm(hi, l, 0x05010400u);  // codes 0 1 2 3
+        hi = __builtin_amdgcn_perm(hi, l, 0x07030602u);  // codes 4 5 6 7
+      }
+      if constexpr (e4 >= 2) {
+        const f16x2 q = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(half ? hi : lo, 512.0f, e4 == 3);
+        out[EL - 2 - 2 * half] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(s, q, b));
+      }
+    } else if constexpr (!F16) {
+      const float v = __builtin_fmaf(s, (float)((w[half] >> (8 * e4)) & 0xffu), b);
+      if constexpr (EL % 2 == 0) f = v;
+      else out[EL / 2] = pack_bf16x2(f, v);
+    } else {
+      constexpr int pair = EL / 2;
+      if constexpr (EL % 2 == 0)
+        p16 = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, w[half], pair % 2 ? 0x04030402u : 0x04010400u)) -
+              f16x2{(_Float16)1024.0f, (_Float16)1024.0f};
+      else
+        out[pair] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(s, p16, b));
+    }
+  }
+};
+
+// Tile of BM = 64, 128 or 256 rows. LDS and registers are kept to 48, 80 and
+// 144 KB and 80, 128 and 256 registers, so that three, two and one workgroups
+// share a compute unit: one covers the other's load latency, barriers and
+// epilogue. WV = 4 (64-row tiles only) halves the weight rows of a tile (128:
+// 64 gate and 64 up rows, or 128 down rows) for twice the tiles, where 8-wave
+// tiles would leave compute units idle (a few experts or a few output
+// columns: Granite decode batches, a dense matrix); 40 KB of LDS.
+template <int BM, int WV>
+constexpr int wr_waves_per_simd() { return BM == 64 ? 4 : 2; }
+
+template <int BM, int MODE, int BITS, bool F16, int WV, bool FEW = false>
+__global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM, WV>())) void ggemm_wr_kernel(GgArgs args) {
   constexpr int WAVES = WV, BN = 32 * WV;
   constexpr int MB = BM / 16;                     // 16-row blocks per wave
   constexpr int OUT_COLS = MODE == kGgGateUp ? BN / 2 : BN;
   constexpr int LA = BM / (4 * WAVES);            // 4-row (1 KB) copies per wave per super-step
-  static_assert(WV == 8 || (WV == 4 && BM == 64), "8 waves, or 4 with 64-row tiles");
+  static_assert(WV == 8 || (WV == 4 && BM <= 128), "8 waves, or 4 with 64- and 128-row tiles");
   static_assert(LA >= 1, "every wave copies activation rows");
   constexpr int SROW = 136;                       // epilogue staging row stride (128 columns + 16 B)
   constexpr int HALF_ROWS = BM / 2;               // staged rows per activation stage
@@ -583,11 +670,14 @@ __global__ __launch_bounds__(WV * 64, BM == 64 ? (WV == 8 ? 2 : 3) : 1) void gge
   static_assert(HALF_ROWS * SROW <= BM * BK2, "epilogue staging fits a stage");
   using op_t = op8_t<F16>;
   using f16tag = std::integral_constant<bool, F16>;
+  using D8 = Deq8<BITS, F16>;
+  using sb_t = typename D8::sb_t;
+  constexpr int RL = BITS / 4;                    // 16-byte raw loads per weight row and super-step
+  constexpr int SBH = BN * 8;                     // scales (or biases) of the tile's rows, 8 groups
 
   __shared__ __attribute__((aligned(16))) uint16_t sA0[BM * BK2];
   __shared__ __attribute__((aligned(16))) uint16_t sA1[BM * BK2];
-  __shared__ __attribute__((aligned(16))) uint16_t sSc[BN * 32];
-  __shared__ __attribute__((aligned(16))) uint16_t sBi[BN * 32];
+  __shared__ __attribute__((aligned(16))) uint16_t sSb[2 * 2 * SBH];  // [ring slot][scale, bias][row][8 groups]
   // Tile prefix, XCD bounds and expert index: in activation stage 1, first
   // written after the prologue's barrier.
   int* const s_tiles = reinterpret_cast<int*>(sA1);
@@ -690,7 +780,7 @@ __global__ __launch_bounds__(WV * 64, BM == 64 ? (WV == 8 ? 2 : 3) : 1) void gge
 
   // ---- weights ----
   const int g4 = lane >> 4;                       // k quarter of the super-step
-  const uint32_t qrow = (uint32_t)args.Kin / 2, srow = (uint32_t)G * 2;
+  const uint32_t qrow = (uint32_t)args.Kin * BITS / 8, srow = (uint32_t)G * 2;
   __amdgpu_buffer_rsrc_t rbq[2];
   uint32_t b_qoff[2];
   int trow[2];                                    // weight row within the tile (0..255)
@@ -700,86 +790,67 @@ __global__ __launch_bounds__(WV * 64, BM == 64 ? (WV == 8 ? 2 : 3) : 1) void gge
     trow[j] = MODE == kGgGateUp ? j * (BN / 2) + 16 * wave + (lane & 15) : 32 * wave + 16 * j + (lane & 15);
     const int bn = MODE == kGgGateUp ? n0 + 16 * wave + (lane & 15) : n0 + 32 * wave + 16 * j + (lane & 15);
     rbq[j] = gg_rsrc(reinterpret_cast<const char*>(bm.q) + (size_t)e * args.N * qrow, (uint32_t)args.N * qrow);
-    b_qoff[j] = bn < args.N ? (uint32_t)bn * qrow + 16u * g4 : kOob;
+    b_qoff[j] = bn < args.N ? (uint32_t)bn * qrow + 4u * BITS * g4 : kOob;
   }
-  auto bload = [&](uint4* raw, int kt) {
+  auto bload = [&](uint4 (*raw)[RL], int kt) {
     const bool live = kt < KT;
 #pragma unroll
     for (int j = 0; j < 2; ++j)
-      raw[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(live ? rbq[j] : rnull, b_qoff[j], kt * 64, 0));
+#pragma unroll
+      for (int r = 0; r < RL; ++r)
+        raw[j][r] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(live ? rbq[j] : rnull, b_qoff[j] + 16 * r, kt * 16 * BITS, 0));
   };
 
-  // Scales and biases of the tile's rows, copied once: HALVES contiguous row
-  // ranges, each at a 1 KB-aligned offset, row r of a range at r * 2G bytes.
-  // sb_read reads one group of 16 consecutive rows per instruction; at a row
-  // stride of 2G bytes those rows share 2 to 4 banks (32 or 64 banks of 4
-  // bytes). The layouts move row r's group-pair dword d to d ^ sw(r):
-  //  * kSbPlain: sw = 0, copied as contiguous 16-byte pieces;
-  //  * kSbDword: sw(r) = (r G / 64) mod (G/2) for G/2 a power of two, which
-  //    puts the 16 rows in 16 banks; copied with 4-byte LDS-DMA, the swizzle
-  //    applied to the source offsets;
-  //  * kSbChunk (G = 16 or 32): 16-byte pieces of a row swapped,
-  //    sw(r) = 4 ((r / 4) mod (G/8)): 2 rows per bank at worst, and the copy
-  //    stays 16-byte LDS-DMA.
-  constexpr int HALVES = MODE == kGgGateUp ? 2 : 1;
-  constexpr int HROWS = BN / HALVES;
-  const int GH = G / 2;                           // group-pair dwords per row
-  const int CH = G / 8;                           // 16-byte pieces per row
-  const int lay = args.sb_layout;
-  const int swm = (GH & (GH - 1)) == 0 ? GH - 1 : 0;
-  auto sb_swz = [&](int r) {
-    return lay == kSbDword ? ((r * G) >> 6) & swm : lay == kSbChunk ? ((r >> 2) & (CH - 1)) << 2 : 0;
-  };
-  const int hbytes = HROWS * G * 2;
-  const int hs = (hbytes + 1023) & ~1023;
-#pragma unroll
-  for (int h = 0; h < HALVES; ++h) {
-    const tfm_affine& bm = h ? args.wb : args.wa;
-    const size_t ebase = (size_t)e * args.N;
-    const auto rs = gg_rsrc(static_cast<const char*>(bm.scales) + ebase * srow, (uint32_t)args.N * srow);
-    const auto rb = gg_rsrc(static_cast<const char*>(bm.biases) + ebase * srow, (uint32_t)args.N * srow);
-    const uint32_t g0 = (uint32_t)n0 * srow;
-    if (lay == kSbDword) {
-      for (int c = wave; c * 256 < hbytes; c += WAVES) {
-        const int p = 64 * c + lane;              // destination dword of the range
-        const int r = p / GH, x = p - r * GH;
-        const uint32_t src = 4 * p < hbytes ? g0 + (uint32_t)r * srow + 4u * (uint32_t)(x ^ sb_swz(r)) : kOob;
-        lds_dma4(rs, sSc + (h * hs + c * 256) / 2, src);
-        lds_dma4(rb, sBi + (h * hs + c * 256) / 2, src);
-      }
+  // Scales and biases: chunk c holds groups 8c..8c+7 (super-steps 4c..4c+3) of
+  // the tile's BN rows, 16 bytes a row, in ring slot c % 2. The first half of
+  // the waves copies scales, the second biases, 64 rows each: one 16-byte
+  // LDS-DMA per wave and chunk. Rows of G groups not a multiple of 8 are only
+  // 4-byte aligned and take four 4-byte copies. A row's last chunk may read
+  // past its groups (the next row's, never used, or zeros past the matrix).
+  // Loaded straight into registers instead, as 2-byte values of 64 rows at a
+  // time, they cost as much as the packed codes; kept for the whole input
+  // width (32 KB at 2048) they cost 128-row tiles a workgroup per compute unit.
+  const int sw = wave % (WAVES / 2);              // rows 64 sw .. 64 sw + 63 of the tile
+  const bool sbias = wave >= WAVES / 2, sup = MODE == kGgGateUp && 64 * sw >= BN / 2;
+  const tfm_affine& sm = sup ? args.wb : args.wa;
+  const auto rsb = gg_rsrc(static_cast<const char*>(sbias ? sm.biases : sm.scales) + (size_t)e * args.N * srow,
+                           (uint32_t)args.N * srow);
+  const int sn0 = n0 + 64 * sw - (sup ? BN / 2 : 0);  // matrix row of the first
+  const bool sb16 = (G & 7) == 0;
+  auto sb_copy = [&](int c) {
+    uint16_t* const dst = sSb + ((c & 1) * 2 + (sbias ? 1 : 0)) * SBH + 64 * 8 * sw;
+    const bool live = 8 * c < G;
+    if (sb16) {
+      const int n = sn0 + lane;
+      lds_dma16(rsb, dst, live && n < args.N ? (uint32_t)n * srow + 16u * c : kOob, 0);
     } else {
-      for (int c = wave; c * 1024 < hbytes; c += WAVES) {
-        uint32_t src = g0 + c * 1024 + lane * 16;
-        if (lay == kSbChunk) {
-          const int p = 64 * c + lane;            // destination 16-byte piece of the range
-          const int r = p / CH, x = p - r * CH;
-          src = 16 * p < hbytes ? g0 + (uint32_t)r * srow + 16u * (uint32_t)(x ^ (sb_swz(r) >> 2)) : kOob;
-        }
-        lds_dma16(rs, sSc + (h * hs + c * 1024) / 2, src, 0);
-        lds_dma16(rb, sBi + (h * hs + c * 1024) / 2, src, 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {               // dword 64 i + lane: row 16 i + lane / 4, pair lane % 4
+        const int n = sn0 + 16 * i + (lane >> 2);
+        lds_dma4(rsb, dst + 128 * i, live && n < args.N ? (uint32_t)n * srow + 16u * c + 4u * (lane & 3) : kOob);
       }
     }
-  }
-  int sidx[2], ssw[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    sidx[j] = (trow[j] / HROWS) * (hs / 2) + (trow[j] % HROWS) * G;
-    ssw[j] = sb_swz(trow[j] % HROWS);
-  }
+  };
   // scale and bias of super-step kt for both rows (past the end: last group)
-  auto sb_read = [&](float* sc, float* bi, int kt) {
+  auto sb_read = [&](sb_t* sc, sb_t* bi, int kt) {
     int g = 2 * kt + (g4 >> 1);
     g = g < G ? g : G - 1;
+    const uint16_t* const p = sSb + ((g >> 3) & 1) * 2 * SBH + (g & 7);
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      const int o = sidx[j] + 2 * ((g >> 1) ^ ssw[j]) + (g & 1);
-      sc[j] = st2f<F16>(sSc[o]);
-      bi[j] = st2f<F16>(sBi[o]);
+      sc[j] = D8::sb(p[trow[j] * 8]);
+      bi[j] = D8::sb(p[trow[j] * 8 + SBH]);
     }
   };
-  auto deq = [&](op_t* b, const uint4* raw, const float* sc, const float* bi, int s) {
+  auto deq = [&](op_t* b, uint4 (*raw)[RL], const sb_t* sc, const sb_t* bi) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) b[j] = __builtin_bit_cast(op_t, dequant_word<F16>(word_of(raw[j], s), sc[j], bi[j]));
+    for (int j = 0; j < 2; ++j) {
+      D8 d;
+      uint32_t o[4];
+      const uint32_t* w = reinterpret_cast<const uint32_t*>(&raw[j][0]);
+      static_for<0, 8>([&](auto el_) { d.template slice<decltype(el_)::value>(w, sc[j], bi[j], o); });
+      b[j] = __builtin_bit_cast(op_t, make_uint4(o[0], o[1], o[2], o[3]));
+    }
   };
 
   f32x4_t acc[MB][2];
@@ -805,8 +876,8 @@ __global__ __launch_bounds__(WV * 64, BM == 64 ? (WV == 8 ? 2 : 3) : 1) void gge
   // lane offset is made opaque per super-step so that the four per-sub-step
   // addresses are formed there instead of being held across the loop.
   const uint32_t a_lane = (uint32_t)((lane & 15) * BK2 * 2 + (((4 * g4) ^ (lane & 15)) << 4));
-  auto compute = [&](auto mbl_tag, const uint16_t* A, op_t* b, const uint4* rc, const float* sc,
-                     const float* bic, const uint4* rn, const float* sn, const float* bin, uint16_t* An,
+  auto compute = [&](auto mbl_tag, const uint16_t* A, op_t* b, uint4 (*rc)[RL], const sb_t* sc,
+                     const sb_t* bic, uint4 (*rn)[RL], const sb_t* sn, const sb_t* bin, uint16_t* An,
                      int ktn, auto after_copy) __attribute__((always_inline)) {
     constexpr int MBL = decltype(mbl_tag)::value;
     constexpr int NQ = 4 * MBL, D = 3, R = D + 1;
@@ -816,8 +887,7 @@ __global__ __launch_bounds__(WV * 64, BM == 64 ? (WV == 8 ? 2 : 3) : 1) void gge
     static_assert(STEP * (NC - 1) < NQ, "every copy is issued");
     op_t af[R];
     uint32_t nbw[2][4];                           // next B operand, packed pairs
-    uint32_t lo[2], hi[2];                        // nibble bytes of the word being dequantised
-    float f[16];
+    D8 dq[2];
     uint32_t al = a_lane;
     asm volatile("" : "+v"(al));
     const char* const Ab = reinterpret_cast<const char*>(A);
@@ -834,24 +904,15 @@ __global__ __launch_bounds__(WV * 64, BM == 64 ? (WV == 8 ? 2 : 3) : 1) void gge
       if constexpr (q + D < NQ) rd(std::integral_constant<int, q + D>{});
       acc[i][0] = mfma16(af[q % R], b[0], acc[i][0], f16tag{});
       acc[i][1] = mfma16(af[q % R], b[1], acc[i][1], f16tag{});
-      // Slice of the next sub-step's B operand: codes c0..c1-1 of the 16
-      // (code c: row j = c / 8, element c % 8 of word s + 1, or word 0 of
-      // the next super-step's raw weights).
+      // Slices of the next sub-step's B operand: slice c of 16 is slice c % 8
+      // of row c / 8 (word(s) s + 1, or the first of the next super-step's raw
+      // weights).
       constexpr int c0 = 16 * i / MBL, c1 = 16 * (i + 1) / MBL;
       static_for<c0, c1>([&](auto c_) {
         constexpr int c = decltype(c_)::value, j = c / 8, el = c % 8;
-        const uint32_t* rw = s < 3 ? reinterpret_cast<const uint32_t*>(&rc[j]) : reinterpret_cast<const uint32_t*>(&rn[j]);
-        const float scj = s < 3 ? sc[j] : sn[j], bij = s < 3 ? bic[j] : bin[j];
-        if constexpr (el == 0) {
-          const uint32_t w = rw[s < 3 ? s + 1 : 0];
-          lo[j] = w & 0x0f0f0f0fu;
-          hi[j] = (w >> 4) & 0x0f0f0f0fu;
-          asm("" : "+v"(lo[j]));
-          asm("" : "+v"(hi[j]));
-        }
-        const uint32_t src = (el & 1) ? hi[j] : lo[j];
-        f[c] = __builtin_fmaf(scj, (float)((src >> (8 * (el >> 1))) & 0xffu), bij);
-        if constexpr (el & 1) nbw[j][el >> 1] = pack_st2<F16>(f[c - 1], f[c]);
+        constexpr int w0 = s < 3 ? RL * (s + 1) : 0;
+        const uint32_t* rw = (s < 3 ? reinterpret_cast<const uint32_t*>(&rc[j][0]) : reinterpret_cast<const uint32_t*>(&rn[j][0])) + w0;
+        dq[j].template slice<el>(rw, s < 3 ? sc[j] : sn[j], s < 3 ? bic[j] : bin[j], nbw[j]);
       });
       if constexpr (i == MBL - 1) {
 #pragma unroll
@@ -873,18 +934,39 @@ __global__ __launch_bounds__(WV * 64, BM == 64 ? (WV == 8 ? 2 : 3) : 1) void gge
   // only for that copy (the vector memory counter retires in issue order), so
   // they stay in flight across it. The products and their order are those of
   // the loop below.
-  if (FEW && rows_valid <= 16 && (KT & 3) == 0) {
-    if constexpr (FEW) {
-      static_assert(BM == 64, "few-row tiles are 64-row tiles");
-      uint4 rw[4][2];                             // raw weights of super-step k in slot k % 4
-      float fsc[2][2], fbi[2][2];                 // scales and biases of super-step k in set k % 2
+  // Live row blocks (uniform over the workgroup): in steps of four of 16
+  // blocks, of two of 8; with 64-row tiles 1, 2 or 4 (16, 32 or 64 rows).
+  auto by_live = [&](auto f) __attribute__((always_inline)) {
+    if constexpr (MB == 16) {
+      if (rows_valid > 192) f(std::integral_constant<int, 16>{});
+      else if (rows_valid > 128) f(std::integral_constant<int, 12>{});
+      else if (rows_valid > 64) f(std::integral_constant<int, 8>{});
+      else f(std::integral_constant<int, 4>{});
+    } else if constexpr (MB == 8) {
+      if (rows_valid > 96) f(std::integral_constant<int, 8>{});
+      else if (rows_valid > 64) f(std::integral_constant<int, 6>{});
+      else if (rows_valid > 32) f(std::integral_constant<int, 4>{});
+      else f(std::integral_constant<int, 2>{});
+    } else {
+      if (rows_valid > 32) f(std::integral_constant<int, 4>{});
+      else if (rows_valid > 16) f(std::integral_constant<int, 2>{});
+      else f(std::integral_constant<int, 1>{});
+    }
+  };
+  constexpr bool AHEAD = FEW;
+  if (AHEAD && (BM == 128 || rows_valid <= 16) && (KT & 3) == 0) {
+    if constexpr (AHEAD) {
+      uint4 rw[4][2][RL];                         // raw weights of super-step k in slot k % 4
+      sb_t fsc[2][2], fbi[2][2];                  // scales and biases of super-step k in set k % 2
       op_t fb[2];
+      sb_copy(0);
       a_copy(sA0, 0);
       bload(rw[0], 0);
       bload(rw[1], 1);
       __syncthreads();  // scale copies and stage 0 complete and visible
       sb_read(fsc[0], fbi[0], 0);
-      deq(fb, rw[0], fsc[0], fbi[0], 0);
+      deq(fb, rw[0], fsc[0], fbi[0]);
+      auto ahead_loop = [&](auto mbl_tag) __attribute__((always_inline)) {
       for (int kt0 = 0; kt0 < KT; kt0 += 4) {
         static_for<0, 4>([&](auto q_) {
           constexpr int q = decltype(q_)::value, c = q % 2, n = 1 - c;
@@ -892,33 +974,45 @@ __global__ __launch_bounds__(WV * 64, BM == 64 ? (WV == 8 ? 2 : 3) : 1) void gge
           uint16_t* const A = c == 0 ? sA0 : sA1;
           uint16_t* const An = c == 0 ? sA1 : sA0;
           sb_read(fsc[n], fbi[n], kt + 1);
+          if constexpr (q == 0) sb_copy(kt0 / 4 + 1);
           __builtin_amdgcn_sched_barrier(0);
-          compute(std::integral_constant<int, 1>{}, A, fb, rw[q], fsc[c], fbi[c], rw[(q + 1) % 4], fsc[n],
+          compute(mbl_tag, A, fb, rw[q], fsc[c], fbi[c], rw[(q + 1) % 4], fsc[n],
                   fbi[n], An, kt + 1, [&] { bload(rw[(q + 2) % 4], kt + 2); });
-          // This wave's copy into An is done (only the two weight loads
-          // issued after it may be outstanding), then every wave's.
-          asm volatile("s_waitcnt vmcnt(2)\n\ts_barrier" ::: "memory");
+          // This wave's copies are done (only the 2 RL weight loads issued
+          // after them may be outstanding), then every wave's.
+          if constexpr (RL == 1)
+            asm volatile("s_waitcnt vmcnt(2)\n\ts_barrier" ::: "memory");
+          else
+            asm volatile("s_waitcnt vmcnt(4)\n\ts_barrier" ::: "memory");
         });
       }
+      };
+      if constexpr (FEW) ahead_loop(std::integral_constant<int, 1>{});
+      else by_live(ahead_loop);
     }
   } else {
   // ---- prologue ----
-  uint4 r0[2], r1[2];
-  float sc0[2], bi0[2], sc1[2], bi1[2];
+  uint4 r0[2][RL], r1[2][RL];
+  sb_t sc0[2], bi0[2], sc1[2], bi1[2];
   op_t bop[2];
+  sb_copy(0);
   a_copy(sA0, 0);
   bload(r0, 0);
   __syncthreads();  // scale copies and stage 0 complete and visible
   sb_read(sc0, bi0, 0);
-  deq(bop, r0, sc0, bi0, 0);
+  deq(bop, r0, sc0, bi0);
 
   // Super-step S: load the raw weights of S+1 and read its scales, compute
   // (copying S+1 into the other stage on the way), barrier. With an odd
-  // count the loop runs one more super-step on zero activations.
+  // count the loop runs one more super-step on zero activations. Scale chunk
+  // c + 1 is requested in super-step 4c: the last read of its ring slot's
+  // old chunk c - 1 was before the barrier that ended super-step 4c - 2, and
+  // its first read comes in super-step 4c + 3.
   auto main_loop = [&](auto mbl_tag) {
     for (int kt = 0; kt < KT; kt += 2) {
       bload(r1, kt + 1);
       sb_read(sc1, bi1, kt + 1);
+      if ((kt & 3) == 0) sb_copy(kt / 4 + 1);
       __builtin_amdgcn_sched_barrier(0);
       compute(mbl_tag, sA0, bop, r0, sc0, bi0, r1, sc1, bi1, sA1, kt + 1, [] {});
       __syncthreads();
@@ -929,33 +1023,7 @@ __global__ __launch_bounds__(WV * 64, BM == 64 ? (WV == 8 ? 2 : 3) : 1) void gge
       __syncthreads();
     }
   };
-  // Live row blocks (uniform over the workgroup), in steps of four (with
-  // 64-row tiles: 1, 2 or 4).
-  const int live = min(MB, ((rows_valid + 63) / 64) * 4);
-  if constexpr (MB == 16) {
-    if (live == 16)
-      main_loop(std::integral_constant<int, 16>{});
-    else if (live == 12)
-      main_loop(std::integral_constant<int, 12>{});
-    else if (live == 8)
-      main_loop(std::integral_constant<int, 8>{});
-    else
-      main_loop(std::integral_constant<int, 4>{});
-  } else if constexpr (MB == 8) {
-    if (live == 8)
-      main_loop(std::integral_constant<int, 8>{});
-    else
-      main_loop(std::integral_constant<int, 4>{});
-  } else {
-    // 64-row tiles (few routes per expert): one or two live blocks when the
-    // tile holds at most 16 or 32 rows, so that empty rows cost no MFMAs.
-    if (rows_valid <= 16)
-      main_loop(std::integral_constant<int, 1>{});
-    else if (rows_valid <= 32)
-      main_loop(std::integral_constant<int, 2>{});
-    else
-      main_loop(std::integral_constant<int, 4>{});
-  }
+  by_live(main_loop);
   }
 
   // ---- epilogue ----
@@ -1015,8 +1083,6 @@ static int tile_override() {
   return v;
 }
 
-// Tile rows of the down GEMM alone (TFM_GGEMM_DOWN_TILE=64/128/256, for
-// measurement; TFM_GGEMM_TILE takes precedence); 0 when unset.
 static int down_tile_override() {
   static int v = [] {
     const char* s = std::getenv("TFM_GGEMM_DOWN_TILE");
@@ -1026,6 +1092,16 @@ static int down_tile_override() {
   return v;
 }
 
+static int waves_override() {
+  static const int v = [] {
+    const char* s = std::getenv("TFM_GGEMM_WAVES");
+    const int n = s ? std::atoi(s) : 0;
+    return n == 4 || n == 8 ? n : 0;
+  }();
+  return v;
+}
+
+// Tile rows of ggemm_kernel.
 static bool use_tall(int64_t n_routes, int E) {
   const int o = tile_override();
   if (o == 256) return true;
@@ -1044,52 +1120,70 @@ static int gg_device_cus() {
   return cus;
 }
 
-// Tile rows of the weights-in-registers kernel (TFM_GGEMM_TILE=64/128/256
-// forces one), from the average routes per expert a = n_routes / E and the
-// tile count, with every expert's routes taken as a:
-//  * 64 while a <= 56: every m-tile streams its expert's weights again, so
-//    64-row tiles pay only while few experts pass 64 routes (OLMoE 33-384
-//    tokens 12% faster than 128-row tiles, level at 512, 9% slower at 768;
-//    Granite 256 tokens, a = 51: 58.6 against 62.6 us per layer);
-//  * 256 from a = 208: a 256-row tile dequantises its weights once for twice
-//    the rows (OLMoE 1792 tokens, a = 224: 309 against 319 us; 2048 tokens:
-//    305 against 331; at a = 192, 1536 tokens, 128-row tiles win, 265
-//    against 277);
-//  * 256 below that when 256-row tiles fit one round of the compute units and
-//    128-row tiles do not (Granite, 4 gate/up column tiles: 768 tokens,
-//    a = 154, 84.4 against 98.6 us; at 512 tokens both fit, and 128-row tiles
-//    win, 70.7 against 73.1);
-//  * else 128;
-//  * with few experts and output columns (E x col_tiles below a quarter of
-//    the compute units: a dense matrix, E = 1), the largest tile whose count
-//    fills the compute units, else 64 (OLMoE q_proj at 512 rows has 16
-//    256-row tiles and 64 64-row ones).
-// col_tiles: 256-row weight tiles across the output (gate/up: gate and up
-// rows together).
-static int wr_tile_rows(int64_t n_routes, int E, int64_t col_tiles, bool down) {
-  const int o = tile_override();
-  if (o == 64 || o == 128 || o == 256) return o;
-  if (4 * E * col_tiles < gg_device_cus()) {
-    const int64_t cus = gg_device_cus();
-    for (int bm = 256; bm >= 128; bm /= 2)
-      if ((n_routes + (int64_t)E * bm - 1) / ((int64_t)E * bm) * E * col_tiles >= cus) return bm;
-    return 64;
-  }
-  if (n_routes <= (int64_t)E * 56) return 64;
-  // The down GEMM keeps 64-row tiles up to 128 routes per expert: two
-  // workgroups per compute unit overlap one's epilogue with the other's main
-  // loop. Down GEMM, 64- against 128-row tiles: OLMoE 512 tokens 40.7 against
-  // 42.8 us, 768 tokens 49.6 against 49.8, 1024 tokens 61.1 against 66.7;
-  // Granite 384 tokens 17.4 against 16.4, 512 tokens 18.1 against 18.1,
-  // 640 tokens 23.8 against 29.0; at OLMoE 2048 tokens (256 routes per
-  // expert) 105.0 against 100.9 on 256-row tiles.
-  if (down && n_routes <= (int64_t)E * 128) return 64;
-  if (n_routes >= (int64_t)E * 208) return 256;
-  const int64_t m128 = (n_routes + (int64_t)E * 128 - 1) / ((int64_t)E * 128);
-  const int64_t m256 = (n_routes + (int64_t)E * 256 - 1) / ((int64_t)E * 256);
+// Tile of the weights-in-registers kernel: rows BM and waves WV.
+struct WrTile {
+  int bm, wv;
+};
+
+// Chosen from the average routes per expert a = n_routes / E and the number
+// of 256-weight-row column tiles (gate/up: gate and up rows together; `wide`:
+// at least one a compute unit over the experts, as OLMoE's and unlike
+// Granite's gate/up). Kernel us at OLMoE (64 experts, 2048 -> 2 x 1024 -> 2048)
+// and Granite (40 experts, 1536 -> 2 x 512 -> 1536) sizes, as rows x waves:
+//  * A dense matrix (few experts and columns): the largest tile whose count
+//    fills the compute units, else 64 x 4 (2048 x 2048 linear: 1024 rows 64x4
+//    19.1, 128x4 23.7; 2048 rows 28.4 and 26.4).
+//  * Down. 64 x 4 up to a = 44 (OLMoE 300 tokens, a = 38: 29.2 against 32.8 on
+//    128x4; 400 tokens: 34.7 and 34.2), then 128 x 4 (512 tokens 38.2 against
+//    42.0 on 64x4 and 40.0 on 128x8; Granite 1024 tokens 27.6, 28.3 on 256x8;
+//    2800 tokens 62.1 and 68.2): two workgroups a compute unit overlap one's
+//    epilogue with the other's main loop. 256 x 8 from a = 448 where the input
+//    is at least 1024 wide, so that the main loop outweighs the epilogue
+//    (OLMoE 2800 tokens, a = 350: 131.4 on 128x4, 132.6 on 256x8; 4000 tokens:
+//    181.2 and 173.7; Granite, 512 wide, 4000 tokens: 85.5 and 91.6).
+//  * Gate/up and gathered products. 64 rows up to a = 44 wide, 56 otherwise
+//    (OLMoE 300 tokens 49.0 against 54.6 on 128x8, 400 tokens 66.0 and 56.7;
+//    Granite 256 tokens, a = 51, 21.8 and 23.7; 8-bit codes 400 tokens 63.0
+//    and 73.6, so to a = 56 there), with 8 waves while that gives two tiles a
+//    compute unit and most experts have a route, else 4 (8-bit codes at 8
+//    tokens 39.5 against 47.4, at 20 tokens 53.8 and 53.5).
+//    128 rows to a = 232 wide (1700 tokens, a = 212: 138.8 against 153.3 on
+//    256x8; 2048 tokens, a = 256: 170.9 and 160.5), 480 otherwise (Granite
+//    1500 tokens, a = 300: 54.0 and 62.0; 2800, a = 560: 93.7 and 84.9): the
+//    256-row tile dequantises its weights once for twice the rows, but with
+//    few tiles its last round leaves much of the chip idle. Eight waves while
+//    an expert has one m-tile (512 tokens 61.7 against 64.4 on 128x4; half
+//    58.0 and 62.6), four above (900 tokens 97.4 against 102.2; Granite 2048
+//    71.8 and 78.3).
+// TFM_GGEMM_TILE=64/128/256 forces the rows, TFM_GGEMM_DOWN_TILE those of the
+// down GEMM alone (TFM_GGEMM_TILE takes precedence), TFM_GGEMM_WAVES=4/8 the
+// waves.
+static WrTile wr_tile(int64_t n_routes, int E, int64_t cols, int kin, int mode, int bits) {
   const int64_t cus = gg_device_cus();
-  if (E * m128 * col_tiles > cus && E * m256 * col_tiles <= cus) return 256;
-  return 128;
+  auto mtiles = [&](int bm) { return (n_routes + (int64_t)E * bm - 1) / ((int64_t)E * bm); };
+  auto pick = [&]() -> WrTile {
+    if (4 * E * cols < cus) {
+      if (E * mtiles(256) * cols >= cus) return {256, 8};
+      if (E * mtiles(128) * cols * 2 >= cus) return {128, 4};
+      return {64, 4};
+    }
+    const bool wide = E * cols >= cus;
+    if (mode == kGgDown) {
+      if (n_routes <= (int64_t)E * (bits == 8 ? 56 : 44)) return {64, 4};
+      if (n_routes >= (int64_t)E * 448 && kin >= 1024) return {256, 8};
+      return {128, 4};
+    }
+    if (n_routes <= (int64_t)E * (wide && bits == 4 ? 44 : 56))
+      return {64, n_routes > 2 * E && E * mtiles(64) * cols >= 2 * cus ? 8 : 4};
+    if (n_routes >= (int64_t)E * (wide ? 232 : 480)) return {256, 8};
+    return {128, n_routes <= (int64_t)E * 104 ? 8 : 4};
+  };
+  WrTile t = pick();
+  int bm = tile_override();
+  if (bm != 64 && bm != 128 && bm != 256) bm = mode == kGgDown ? down_tile_override() : 0;
+  if (bm && bm != t.bm) t = {bm, bm == 64 ? 4 : 8};
+  if (waves_override() && t.bm != 256) t.wv = waves_override();
+  return t;
 }
 
 static unsigned grid_for(int64_t n_routes, int E, int BM, int NT) {
@@ -1111,38 +1205,6 @@ static void launch_one(const GgArgs& a, int64_t n_routes, int E, hipStream_t s) 
     tfm_launch(ggemm_kernel<BM_, BN_, WAVES_M, WAVES_N, MODE, BITS, F16, false>, grid_for(n_routes, E, BM_, NT), C::THREADS, 0, s, a);
 }
 
-// Waves per workgroup of the 64-row weights-in-registers tiles
-// (TFM_GGEMM_WAVES=4/8 forces one): 4 (tiles of half the weight rows) while
-// 8-wave tiles number fewer than two per compute unit, else 8. Per layer, 4
-// against 8 waves: Granite decode 32 38.9 against 40.7 us, Granite 64 tokens
-// 40.8 against 42.5; OLMoE 32 tokens (over two tiles per compute unit) 85.7
-// against 75.2. Two-wave tiles measured no faster than four (Granite decode
-// 32: 40.2 us).
-static int wr_waves(int64_t tiles8) {
-  static const int o = [] {
-    const char* s = std::getenv("TFM_GGEMM_WAVES");
-    return s ? std::atoi(s) : 0;
-  }();
-  if (o == 4 || o == 8) return o;
-  return tiles8 < 2 * (int64_t)gg_device_cus() ? 4 : 8;
-}
-
-// Scale/bias layout of ggemm_wr_kernel for an input width (TFM_GGEMM_SB_LAYOUT
-// = 0/1/2 forces kSbPlain/kSbDword/kSbChunk where it applies): kSbChunk at
-// 16 and 32 groups per row, else kSbPlain. Per layer, plain / dword / chunk
-// layouts on one box: OLMoE 4096 tokens (Zipf) 517.7 / 512.5 / 509.8 us
-// (gate/up 274.2 / 268.9 / 267.0), 512 tokens 138.1 / 135.5 / 134.9; Granite
-// 2048 tokens 156.5 / 157.4 / 156.3, decode 32 39.7 / 40.3 / 39.7.
-static int sb_layout(int Kin) {
-  static const int o = [] {
-    const char* s = std::getenv("TFM_GGEMM_SB_LAYOUT");
-    return s ? std::atoi(s) : -1;
-  }();
-  const int G = Kin / BK;
-  if (o == kSbPlain || o == kSbDword) return o;
-  return G == 16 || G == 32 ? kSbChunk : kSbPlain;
-}
-
 // The FEW instance of a 64-row launch (tiles of at most 16 rows keep their
 // weights two super-steps ahead) runs where experts average at most
 // kFewRowsAvg routes, so that most tiles hold at most 16 rows.
@@ -1156,10 +1218,8 @@ static bool use_few_rows(int64_t n_routes, int E) {
   return v == 2 || (v == 1 && n_routes <= (int64_t)E * kFewRowsAvg);
 }
 
-template <int BM, int MODE, bool F16, int WV>
-static void launch_wr_waves(const GgArgs& a_in, int64_t n_routes, int E, hipStream_t s) {
-  GgArgs a = a_in;
-  a.sb_layout = sb_layout(a.Kin);
+template <int BM, int MODE, int BITS, bool F16, int WV>
+static void launch_wr(const GgArgs& a, int64_t n_routes, int E, hipStream_t s) {
   constexpr int OUT_COLS = MODE == kGgGateUp ? 16 * WV : 32 * WV;
   const int NT = (a.N + OUT_COLS - 1) / OUT_COLS;
   // With 256-row tiles an XCD's run of cheap tiles holds more tiles than an
@@ -1167,65 +1227,64 @@ static void launch_wr_waves(const GgArgs& a_in, int64_t n_routes, int E, hipStre
   // 17); workgroups past their XCD's run exit at once.
   unsigned grid = grid_for(n_routes, E, BM, NT);
   if (BM == 256) grid = ((grid / 8 * 29 + 16) / 17 + 2) * 8;
-  // Not for 8-wave half storage: there the ring would cost a workgroup per
-  // compute unit (three waves per SIMD).
-  if constexpr (BM == 64 && !(F16 && WV == 8)) {
+  if constexpr (BM == 64 && BITS == 4) {
     if (use_few_rows(n_routes, E)) {
-      tfm_launch(ggemm_wr_kernel<BM, MODE, F16, WV, true>, grid, WV * 64, 0, s, a);
+      tfm_launch(ggemm_wr_kernel<BM, MODE, BITS, F16, WV, true>, grid, WV * 64, 0, s, a);
       return;
     }
   }
-  tfm_launch(ggemm_wr_kernel<BM, MODE, F16, WV>, grid, WV * 64, 0, s, a);
+  tfm_launch(ggemm_wr_kernel<BM, MODE, BITS, F16, WV>, grid, WV * 64, 0, s, a);
 }
 
-// 4-bit weights, inputs up to 2048 wide and a multiple of 128: weights in
-// registers (ggemm_wr_kernel); otherwise ggemm_kernel.
-template <int BM, int MODE, bool F16>
-static void launch_wr(const GgArgs& a, int64_t n_routes, int E, hipStream_t s) {
-  if constexpr (BM == 64) {
-    constexpr int OUT8 = MODE == kGgGateUp ? 128 : 256;
-    const int wv = wr_waves(grid_for(n_routes, E, BM, (a.N + OUT8 - 1) / OUT8));
-    if (wv == 4) {
-      launch_wr_waves<BM, MODE, F16, 4>(a, n_routes, E, s);
-      return;
-    }
-  }
-  launch_wr_waves<BM, MODE, F16, 8>(a, n_routes, E, s);
-}
-
+// Inputs a multiple of 128 wide: weights in registers (ggemm_wr_kernel);
+// otherwise (odd multiples of 64) ggemm_kernel.
 template <int MODE, int BITS, bool F16>
 static void launch_tile(const GgArgs& a, int64_t n_routes, int E, hipStream_t s) {
-#ifndef GG_NO_WR
-  if constexpr (BITS == 4) {
-    if (a.Kin <= kLdsScaleKin && a.Kin % BK2 == 0) {
-      int bm = wr_tile_rows(n_routes, E, MODE == kGgGateUp ? (2 * (int64_t)a.N + 255) / 256 : ((int64_t)a.N + 255) / 256,
-                            MODE == kGgDown);
-      if (MODE == kGgDown && down_tile_override() && !tile_override()) bm = down_tile_override();
-      switch (bm) {
-        case 256: launch_wr<256, MODE, F16>(a, n_routes, E, s); break;
-        case 64: launch_wr<64, MODE, F16>(a, n_routes, E, s); break;
-        default: launch_wr<128, MODE, F16>(a, n_routes, E, s); break;
-      }
-      return;
-    }
+  if (a.Kin % BK2 == 0) {
+    const WrTile t = wr_tile(n_routes, E, MODE == kGgGateUp ? (2 * (int64_t)a.N + 255) / 256 : ((int64_t)a.N + 255) / 256,
+                             a.Kin, MODE, BITS);
+    if (t.bm == 256) launch_wr<256, MODE, BITS, F16, 8>(a, n_routes, E, s);
+    else if (t.bm == 128 && t.wv == 8) launch_wr<128, MODE, BITS, F16, 8>(a, n_routes, E, s);
+    else if (t.bm == 128) launch_wr<128, MODE, BITS, F16, 4>(a, n_routes, E, s);
+    else if (t.wv == 8) launch_wr<64, MODE, BITS, F16, 8>(a, n_routes, E, s);
+    else launch_wr<64, MODE, BITS, F16, 4>(a, n_routes, E, s);
+    return;
   }
-#endif
   if (use_tall(n_routes, E))
     launch_one<256, 256, 2, 4, MODE, BITS, F16>(a, n_routes, E, s);
   else
     launch_one<128, 256, 2, 4, MODE, BITS, F16>(a, n_routes, E, s);
 }
 
+#define TFM_GG_RUN2(b, t) ggemm_run_##b##_##t
+#define TFM_GG_RUN1(b, t) TFM_GG_RUN2(b, t)
+#define TFM_GG_RUN TFM_GG_RUN1(TFM_GG_BITS, TFM_GG_F16)
+
+void TFM_GG_RUN(int mode, const GgArgs& a, int64_t n_routes, int E, hipStream_t s) {
+  constexpr int BITS = TFM_GG_BITS;
+  constexpr bool F16 = TFM_GG_F16 != 0;
+  switch (mode) {
+    case kGgGateUp: launch_tile<kGgGateUp, BITS, F16>(a, n_routes, E, s); break;
+    case kGgDown: launch_tile<kGgDown, BITS, F16>(a, n_routes, E, s); break;
+    default: launch_tile<kGgPlain, BITS, F16>(a, n_routes, E, s); break;
+  }
+}
+
+#if TFM_GG_MAIN
+void ggemm_run_4_1(int mode, const GgArgs& a, int64_t n_routes, int E, hipStream_t s);
+void ggemm_run_8_0(int mode, const GgArgs& a, int64_t n_routes, int E, hipStream_t s);
+void ggemm_run_8_1(int mode, const GgArgs& a, int64_t n_routes, int E, hipStream_t s);
+
 template <int MODE>
 static void launch_mode(const GgArgs& a, int bits, bool f16, int64_t n_routes, int E, hipStream_t s) {
   if (bits == 8 && f16)
-    launch_tile<MODE, 8, true>(a, n_routes, E, s);
+    ggemm_run_8_1(MODE, a, n_routes, E, s);
   else if (bits == 8)
-    launch_tile<MODE, 8, false>(a, n_routes, E, s);
+    ggemm_run_8_0(MODE, a, n_routes, E, s);
   else if (f16)
-    launch_tile<MODE, 4, true>(a, n_routes, E, s);
+    ggemm_run_4_1(MODE, a, n_routes, E, s);
   else
-    launch_tile<MODE, 4, false>(a, n_routes, E, s);
+    ggemm_run_4_0(MODE, a, n_routes, E, s);
 }
 
 static void check_shapes(int N, int Kin, int bits, int64_t x_rows) {
@@ -1274,5 +1333,7 @@ void launch_ggemm_plain(const uint16_t* x, RowMap rm, const Grouping& g, int64_t
   launch_mode<kGgPlain>(a, bits, f16, n_routes, E, s);
   check_hip(hipGetLastError(), "grouped GEMM plain launch");
 }
+
+#endif  // TFM_GG_MAIN
 
 }  // namespace tfm
