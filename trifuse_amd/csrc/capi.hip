@@ -251,29 +251,6 @@ static bool ds_prefetch() {
   return v;
 }
 
-// Tokens up to which the prefill-path routing runs as two kernels (router
-// logits with one wave per few (token, expert) pairs, then top-k with the
-// chunk histograms) rather than the fused router + top-k kernel, whose
-// 4-token workgroups leave most of the chip idle on small batches. Per
-// layer, fused against split: OLMoE 32 tokens 120.0 against 112.0 us,
-// 128 tokens 174.5 against 168.5, 512 tokens 141.4 against 139.6, 1024
-// tokens 205.9 against 207.5, 4096 tokens (Zipf) 527.6 against 532.0;
-// Granite decode 32 41.6 against 38.1. TFM_ROUTER_SPLIT_MAX_TOKENS overrides.
-static int router_split_max_tokens() {
-  static const int v = [] {
-    const char* s = std::getenv("TFM_ROUTER_SPLIT_MAX_TOKENS");
-    if (!s) return 512;
-    char* end = nullptr;
-    const long n = std::strtol(s, &end, 10);
-    if (!end || end == s || *end != 0 || n < 0 || n > (1 << 30)) {
-      std::fprintf(stderr, "trifuse_moe: ignoring invalid TFM_ROUTER_SPLIT_MAX_TOKENS=%s\n", s);
-      return 512;
-    }
-    return (int)n;
-  }();
-  return v;
-}
-
 static bool fused_decode(const tfm_geometry& g, int64_t R) {
   return R <= 256 && g.hidden_size <= 2048 && g.intermediate_size <= 2048;
 }
@@ -921,9 +898,9 @@ static void moe_forward_body(const tfm_plan* plan, const void* x, int64_t tokens
       launch_dequant_router(f16, weights->router_bits, weights->router_affine, E, H, ws.router_w, s);
       rw = ws.router_w;
     }
-    if (T > router_split_max_tokens())
+    if (R > 256)
       fused_route = launch_router_topk(g.route, f16, static_cast<const uint16_t*>(x), rw, weights->logit_bias,
-                                       T, H, E, K, ws.idx, ws.gates, ws.hist, nullptr, s);
+                                       T, H, E, K, ws.idx, ws.gates, ws.hist, s);
     if (!fused_route)
       launch_router_logits(f16, static_cast<const uint16_t*>(x), rw, weights->logit_bias, (int)tokens, H, E,
                            ws.logits, s);
@@ -943,7 +920,8 @@ static void moe_forward_body(const tfm_plan* plan, const void* x, int64_t tokens
   }
   if (!small_group) {
     StageScope st(TFM_STAGE_GROUP, s);
-    launch_group_scatter(ws.idx, R, E, kTopkTokensPerBlock * K, ws.hist, ws.grp, &ws.hdr->status, s);
+    launch_group_scatter(ws.idx, R, E, (fused_route ? router_topk_tokens(T) : kTopkTokensPerBlock) * K, ws.hist, ws.grp,
+                         &ws.hdr->status, s);
   }
   if (idx_out) launch_copy_i32(ws.idx, idx_out, R, s);
   if (gates_out) launch_copy_i32(reinterpret_cast<const int32_t*>(ws.gates),

@@ -92,156 +92,337 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const uint16_t* __re
 }
 
 // Prefill routing in one pass: router linear, top-k and the chunk histogram
-// for the grouping. A workgroup takes kTopkTokensPerBlock (4) tokens with W
-// waves: every wave keeps their x rows in registers and computes the logits
-// of 1/W of the experts, streaming those router rows (the next one loading
-// while the current one is used), each logit exactly as router_logits_kernel
-// computes it. Then wave t < 4 ranks token t from the logits in LDS with the
-// same wave-level ranking as topk_kernel. Few tokens take W = 8 (each wave
-// waits on a chain of E/8 router-row loads instead of E/4: 512 tokens
-// 21 -> 16 us); many take W = 4, two workgroups per compute unit.
-template <int C, int ROUTE, bool F16, int W>
-__global__ __launch_bounds__(W * 64) void router_topk_kernel(const uint16_t* __restrict__ x,
-                                                          const uint16_t* __restrict__ w,
-                                                          const float* __restrict__ bias, int T,
-                                                          int H, int E, int K,
-                                                          int32_t* __restrict__ idx,
-                                                          float* __restrict__ gates_f32,
-                                                          int32_t* __restrict__ hist,
-                                                          uint16_t* __restrict__ logits_out) {
-  constexpr int TB = kTopkTokensPerBlock;
-  static_assert(TB == 4, "one ranking wave per token");
-  __shared__ uint16_t s_logit[TB][64];
+// for the grouping, 4 or 16 tokens a workgroup of eight waves.
+//
+// The logits run on the matrix cores in their bit-defined order: an fp32 MFMA
+// of k = 1 adds one product to each accumulator with a single rounding
+// (subnormal results included), so a chain of C of them over the elements of
+// lane segment l is the sequential fused multiply-add chain of that segment.
+//  * 4 tokens: v_mfma_f32_4x4x1 (16 blocks: 16 segments of 4 tokens x 4
+//    experts). Wave (m, half) holds segments 16m..16m+15 of half the experts;
+//    lane 4b+i supplies x of token i and w of expert i in segment 16m+b, and
+//    receives the 4 tokens' sums of expert i. The pairwise tree then runs over
+//    the lanes' b (two DPP shifts, two lane-half exchanges that also move token
+//    t to row t), and over m through LDS.
+//  * 16 tokens: v_mfma_f32_16x16x1 (4 blocks: 4 segments of 16 tokens x 16
+//    experts). Wave v holds segments 8v..8v+7 of every expert; lane 16b+i
+//    supplies row i in segment 4q+b of its quad q. The tree's first three
+//    levels are sums of a lane's registers, the last three go through LDS.
+// Wave t then ranks tokens t, t + 8, .. from LDS as topk_kernel does.
+//
+// Operands come through LDS, because a lane's segment is C x 2 contiguous
+// bytes: loaded straight into registers, every 16-byte load of a wave touches
+// 64 separate 64-byte pieces, and the address unit takes about 64 cycles over
+// it (256 such loads a workgroup: 4-token workgroups took 15.8 us however few
+// there were, 11.4 through LDS). The copies read rows contiguously; the slot
+// of a chunk is rotated by its row, so that the 16 lanes of a read pass hit 16
+// bank groups. Router rows are private to a wave, two slots deep.
+//
+// Bound: 2 E H flop per token at 256 flop per clock and compute unit in the
+// 16 x 16 form (the 4 x 4 form measured about a quarter of that), and the E H
+// x 2 bytes of router rows per workgroup from L2. Up to 1024 tokens the 4-token
+// form fills the chip and the few products are not its bound; beyond, 16
+// tokens read the router a quarter as often.
+__device__ __forceinline__ void route_dma16(__amdgpu_buffer_rsrc_t r, uint16_t* dst, uint32_t voff) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, voff, 0, 0, 0);
+#else
+  (void)r; (void)dst; (void)voff;
+#endif
+}
+
+// Ranks token t0 + t of the block from its E logits in LDS and counts its
+// routes (whole wave).
+template <int ROUTE, bool F16>
+__device__ __forceinline__ void rank_token(const uint16_t* row, int64_t tok, int E, int K, int32_t* __restrict__ idx,
+                                           float* __restrict__ gates_f32, int* h) {
+  const int lane = threadIdx.x & 63;
+  float g;
+  int id;
+  if (ROUTE == TFM_ROUTE_OLMOE) {
+    uint16_t gb;
+    id = olmoe_route_wave<F16>(row, E, K, &g, &gb);
+  } else {
+    id = granite_route_wave<F16>(row, E, K, &g);
+  }
+  if (lane < K) {
+    idx[tok * K + lane] = id;
+    gates_f32[tok * K + lane] = g;
+    atomicAdd(&h[id], 1);
+  }
+}
+
+template <int C, int ROUTE, bool F16, int NTW>
+__global__ __launch_bounds__(512) void router_topk4_kernel(const uint16_t* __restrict__ x,
+                                                           const uint16_t* __restrict__ w,
+                                                           const float* __restrict__ bias, int T, int H, int E, int K,
+                                                           int32_t* __restrict__ idx, float* __restrict__ gates_f32,
+                                                           int32_t* __restrict__ hist) {
+  constexpr int SEG = C / 8;                      // 16-byte chunks per lane segment
+  constexpr int TS = 2;                           // expert tiles a step: two MFMA chains
+  constexpr int STEPS = (NTW + TS - 1) / TS;
+  constexpr int PE = 68;                          // padded row of 64 experts
+  constexpr int ROW = 512;                        // a 1 KB row: 64 slots of 8 elements
+  __shared__ __attribute__((aligned(16))) uint16_t s_x[4][4][ROW];
+  __shared__ __attribute__((aligned(16))) uint16_t s_w0[8][4 * TS][ROW];
+  __shared__ __attribute__((aligned(16))) uint16_t s_w1[8][4 * TS][ROW];
   __shared__ int h[65];
+  // After the products the token rows are dead: partial sums, then logits.
+  float (*const part)[4][PE] = reinterpret_cast<float (*)[4][PE]>(&s_x[0][0][0]);
+  uint16_t (*const s_logit)[64] = reinterpret_cast<uint16_t (*)[64]>(&s_x[0][0][0] + 4 * 4 * PE * 2);
+  static_assert(4 * 4 * PE * 4 + 4 * 64 * 2 <= (int)sizeof(s_x), "partial sums and logits fit the token rows");
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   if (tid <= E) h[tid] = 0;
-  const int t0 = blockIdx.x * TB;
-  float xv[TB][C];
-#pragma unroll
-  for (int t = 0; t < TB; ++t) {
-    if (t0 + t < T) {
-      const uint4* src = reinterpret_cast<const uint4*>(x + (int64_t)(t0 + t) * H + lane * C);
-#pragma unroll
-      for (int i = 0; i < C / 8; ++i) {
-        const uint4 v = src[i];
-        xv[t][8 * i + 0] = lo_st<F16>(v.x); xv[t][8 * i + 1] = hi_st<F16>(v.x);
-        xv[t][8 * i + 2] = lo_st<F16>(v.y); xv[t][8 * i + 3] = hi_st<F16>(v.y);
-        xv[t][8 * i + 4] = lo_st<F16>(v.z); xv[t][8 * i + 5] = hi_st<F16>(v.z);
-        xv[t][8 * i + 6] = lo_st<F16>(v.w); xv[t][8 * i + 7] = hi_st<F16>(v.w);
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < C; ++j) xv[t][j] = 0.0f;
-    }
+  const int t0 = blockIdx.x * 4;
+  const int m = wave & 3, e0 = (wave >> 2) * 4 * NTW;
+  const int b = lane >> 2, i4 = lane & 3;
+
+  // Rows past T and past E are beyond their buffers and read as zero.
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(x + (int64_t)t0 * H), (short)0, min(4, T - t0) * H * 2, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(w), (short)0, E * H * 2, 0x00020000);
+  // Chunk (b, s) of a row with index i mod 4 sits in slot (b SEG + s + rot(i))
+  // mod 64; the byte offset within its row of the chunk that lane l copies to
+  // slot l (slots past the segments' chunks get zeros).
+  auto rot = [](int i) { return SEG == 4 ? i : SEG == 2 ? (i & 1) + 8 * (i >> 1) : 4 * i; };
+  auto src = [&](int i, int mm) -> uint32_t {
+    const int c = (lane - rot(i)) & 63;
+    return c < 16 * SEG ? (uint32_t)(16 * mm * SEG + c) * 16u : 0x80000000u;
+  };
+  for (int q = wave; q < 16; q += 8) {
+    const int t = q >> 2, mm = q & 3;
+    route_dma16(rx, &s_x[mm][t][0], (uint32_t)t * H * 2 + src(t, mm));
   }
-  auto wrow = [&](uint4 (&r)[C / 8], int e) {
-    const uint4* src = reinterpret_cast<const uint4*>(w + (int64_t)e * H + lane * C);
+  uint32_t wsrc[4];
 #pragma unroll
-    for (int i = 0; i < C / 8; ++i) r[i] = src[i];
+  for (int i = 0; i < 4; ++i) wsrc[i] = src(i, m);
+  auto copy_w = [&](uint16_t (*dst)[ROW], int step) {
+#pragma unroll
+    for (int r = 0; r < 4 * TS; ++r)
+      route_dma16(rw, dst[r], (uint32_t)(e0 + 4 * TS * step + r) * H * 2 + wsrc[r & 3]);
   };
-  auto logits_of = [&](const uint4 (&r)[C / 8], int e) {
-    float wv[C];
+  copy_w(s_w0[wave], 0);
+  __syncthreads();  // token rows and the first router rows are in LDS
+  if constexpr (STEPS > 1) copy_w(s_w1[wave], 1);
+
+  auto slot = [&](int s) { return ((b * SEG + s + rot(i4)) & 63) * 8; };
+  f32x4_t acc[STEPS * TS];
 #pragma unroll
-    for (int i = 0; i < C / 8; ++i) {
-      wv[8 * i + 0] = lo_st<F16>(r[i].x); wv[8 * i + 1] = hi_st<F16>(r[i].x);
-      wv[8 * i + 2] = lo_st<F16>(r[i].y); wv[8 * i + 3] = hi_st<F16>(r[i].y);
-      wv[8 * i + 4] = lo_st<F16>(r[i].z); wv[8 * i + 5] = hi_st<F16>(r[i].z);
-      wv[8 * i + 6] = lo_st<F16>(r[i].w); wv[8 * i + 7] = hi_st<F16>(r[i].w);
+  for (int n = 0; n < STEPS * TS; ++n) acc[n] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int step = 0; step < STEPS; ++step) {
+    uint16_t (*const ws)[ROW] = step % 2 == 0 ? s_w0[wave] : s_w1[wave];
+    uint4 wr[TS][SEG], xr[SEG];
+#pragma unroll
+    for (int s = 0; s < SEG; ++s) {
+      xr[s] = *reinterpret_cast<const uint4*>(&s_x[m][i4][slot(s)]);
+#pragma unroll
+      for (int n = 0; n < TS; ++n) wr[n][s] = *reinterpret_cast<const uint4*>(&ws[4 * n + i4][slot(s)]);
     }
-    const float be = bias ? bias[e] : 0.0f;
-    float s[TB];
+    // The slot is read before it is copied over.
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (step + 2 < STEPS) copy_w(ws, step + 2);
 #pragma unroll
-    for (int t = 0; t < TB; ++t) {
-      s[t] = 0.0f;
+    for (int j = 0; j < C; ++j) {
+      const uint32_t v = word_of(xr[j >> 3], (j >> 1) & 3);
+      const float xv = j & 1 ? hi_st<F16>(v) : lo_st<F16>(v);
 #pragma unroll
-      for (int j = 0; j < C; ++j) s[t] = __builtin_fmaf(xv[t][j], wv[j], s[t]);
+      for (int n = 0; n < TS; ++n) {
+        const uint32_t u = word_of(wr[n][j >> 3], (j >> 1) & 3);
+        acc[TS * step + n] = __builtin_amdgcn_mfma_f32_4x4x1f32(xv, j & 1 ? hi_st<F16>(u) : lo_st<F16>(u), acc[TS * step + n], 0, 0, 0);
+      }
     }
-    // Row t of the wave holds token t's logit.
-    const float lg = wave_tree_sum64x4(s[0], s[1], s[2], s[3]);
-    if ((lane & 15) == 0) s_logit[lane >> 4][e] = f2st<F16>(bias ? lg + be : lg);
-  };
-  const int epw = (E + W - 1) / W;
-  const int e0 = wave * epw, e1 = min(E, e0 + epw);
-  if (e0 < e1) {  // wave-uniform
-    uint4 ra[C / 8], rb[C / 8];
-    wrow(ra, e0);
-    for (int e = e0; e < e1; e += 2) {
-      if (e + 1 < e1) wrow(rb, e + 1);
-      logits_of(ra, e);
-      if (e + 1 >= e1) break;
-      if (e + 2 < e1) wrow(ra, e + 2);
-      logits_of(rb, e + 1);
+    // Next step's rows (a wave's own copies, in order) have arrived once only
+    // those requested after them may be outstanding.
+    if (step + 2 < STEPS)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * TS) : "memory");
+    else if (step + 1 < STEPS)
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+  __syncthreads();  // every wave is done with the token rows
+#pragma unroll
+  for (int n = 0; n < NTW; ++n) {
+    float v[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      v[t] = acc[n][t];
+      v[t] = dpp_plus<0x104, 0xf>(v[t]);          // row_shl:4  (segment ^ 1), kept by lanes 0-3 and 8-11 of a row
+      v[t] = dpp_plus<0x108, 0xf>(v[t]);          // row_shl:8  (segment ^ 2), kept by lanes 0-3
+    }
+    const float r = row_roots4(v[0], v[1], v[2], v[3]);  // segments ^ 4 and ^ 8; row t: token t
+    if ((lane & 15) < 4) part[m][lane >> 4][e0 + 4 * n + (lane & 15)] = r;
+  }
+  __syncthreads();
+  if (tid < 256) {
+    const int t = tid >> 6, e = tid & 63;
+    if (e < E) {
+      const float lg = (part[0][t][e] + part[1][t][e]) + (part[2][t][e] + part[3][t][e]);
+      s_logit[t][e] = f2st<F16>(bias ? lg + bias[e] : lg);
     }
   }
   __syncthreads();  // every expert's logits of the block's tokens are in LDS
-  const int tok = t0 + wave;
-  if (wave < TB && tok < T) {  // wave-uniform
-    const uint16_t* row = &s_logit[wave][0];
-    if (logits_out && lane < E) logits_out[(int64_t)tok * E + lane] = row[lane];
-    float g;
-    int id;
-    if (ROUTE == TFM_ROUTE_OLMOE) {
-      uint16_t gb;
-      id = olmoe_route_wave<F16>(row, E, K, &g, &gb);
-    } else {
-      id = granite_route_wave<F16>(row, E, K, &g);
-    }
-    if (lane < K) {
-      idx[(int64_t)tok * K + lane] = id;
-      gates_f32[(int64_t)tok * K + lane] = g;
-      atomicAdd(&h[id], 1);
-    }
-  }
+  if (wave < 4 && t0 + wave < T)  // wave-uniform
+    rank_token<ROUTE, F16>(s_logit[wave], (int64_t)t0 + wave, E, K, idx, gates_f32, h);
   __syncthreads();
   if (tid <= E) hist[(int64_t)blockIdx.x * (E + 1) + tid] = h[tid];
 }
 
-template <int C, bool F16>
-static void launch_router_topk_c(int route_kind, const uint16_t* x, const uint16_t* w,
-                                 const float* bias, int T, int H, int E, int K, int32_t* idx,
-                                 float* gates_f32, int32_t* hist, uint16_t* logits_out,
-                                 hipStream_t s) {
-  const unsigned blocks = (unsigned)((T + kTopkTokensPerBlock - 1) / kTopkTokensPerBlock);
-  const bool few = blocks < 512;  // under 2048 tokens: eight waves per workgroup
-  if (route_kind == TFM_ROUTE_OLMOE) {
-    if (few)
-      tfm_launch(router_topk_kernel<C, TFM_ROUTE_OLMOE, F16, 8>, blocks, 512, 0, s, x, w, bias, T, H, E, K, idx, gates_f32,
-                 hist, logits_out);
-    else
-      tfm_launch(router_topk_kernel<C, TFM_ROUTE_OLMOE, F16, 4>, blocks, 256, 0, s, x, w, bias, T, H, E, K, idx, gates_f32,
-                 hist, logits_out);
+template <int C, int ROUTE, bool F16, int NT>
+__global__ __launch_bounds__(512) void router_topk16_kernel(const uint16_t* __restrict__ x,
+                                                            const uint16_t* __restrict__ w,
+                                                            const float* __restrict__ bias, int T, int H, int E, int K,
+                                                            int32_t* __restrict__ idx, float* __restrict__ gates_f32,
+                                                            int32_t* __restrict__ hist) {
+  constexpr int SEG = C / 8;                      // 16-byte chunks per lane segment
+  constexpr int ROW = 256;                        // a wave's 512 bytes of a row: 32 slots of 8 elements
+  constexpr int PE = 68;
+  __shared__ __attribute__((aligned(16))) uint16_t s_r0[8][16][ROW];
+  __shared__ __attribute__((aligned(16))) uint16_t s_r1[8][16][ROW];
+  __shared__ uint16_t s_logit[16][64];
+  __shared__ int h[65];
+  float (*const part)[16][PE] = reinterpret_cast<float (*)[16][PE]>(&s_r0[0][0][0]);  // after the products
+  static_assert(8 * 16 * PE * 4 <= (int)sizeof(s_r0), "partial sums fit a ring slot");
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (tid <= E) h[tid] = 0;
+  const int t0 = blockIdx.x * 16;
+  const int b = lane >> 4, i16 = lane & 15;
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(x + (int64_t)t0 * H), (short)0, min(16, T - t0) * H * 2, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(w), (short)0, E * H * 2, 0x00020000);
+  // 16 rows (tokens, or the experts of tile n) of this wave's 8 segments, two
+  // rows a copy: chunk c of row r in slot (c + r) mod 32.
+  auto copy16 = [&](__amdgpu_buffer_rsrc_t rs, uint16_t (*dst)[ROW], int first) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int r = 2 * k + (lane >> 5);
+      const int c = ((lane & 31) - r) & 31;
+      route_dma16(rs, dst[2 * k], c < 8 * SEG ? (uint32_t)(first + r) * H * 2 + (uint32_t)(8 * wave * SEG + c) * 16u : 0x80000000u);
+    }
+  };
+  auto slot = [&](int q, int s) { return (((4 * q + b) * SEG + s + i16) & 31) * 8; };
+  // Ring order: tokens, then expert tiles 0 .. NT-1. Rows are private to the
+  // wave, so its own wait for its copies is enough.
+  copy16(rx, s_r0[wave], 0);
+  copy16(rw, s_r1[wave], 0);
+  asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+  uint4 xr[2][SEG];
+#pragma unroll
+  for (int q = 0; q < 2; ++q)
+#pragma unroll
+    for (int s = 0; s < SEG; ++s) xr[q][s] = *reinterpret_cast<const uint4*>(&s_r0[wave][i16][slot(q, s)]);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  if constexpr (NT > 1) {
+    copy16(rw, s_r0[wave], 16);
+    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
   } else {
-    if (few)
-      tfm_launch(router_topk_kernel<C, TFM_ROUTE_GRANITE, F16, 8>, blocks, 512, 0, s, x, w, bias, T, H, E, K, idx, gates_f32,
-                 hist, logits_out);
-    else
-      tfm_launch(router_topk_kernel<C, TFM_ROUTE_GRANITE, F16, 4>, blocks, 256, 0, s, x, w, bias, T, H, E, K, idx, gates_f32,
-                 hist, logits_out);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
+  float sum8[NT][4];                              // segments 8 wave .. + 7: token 4 b + r, expert 16 n + i16
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    uint16_t (*const ws)[ROW] = n % 2 == 0 ? s_r1[wave] : s_r0[wave];
+    uint4 wr[2][SEG];
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int s = 0; s < SEG; ++s) wr[q][s] = *reinterpret_cast<const uint4*>(&ws[i16][slot(q, s)]);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot is read before it is copied over
+    if (n + 2 < NT) copy16(rw, ws, 16 * (n + 2));
+    f32x16_t acc[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[q][v] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < C; ++j)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const uint32_t v = word_of(xr[q][j >> 3], (j >> 1) & 3), u = word_of(wr[q][j >> 3], (j >> 1) & 3);
+        acc[q] = __builtin_amdgcn_mfma_f32_16x16x1f32(j & 1 ? hi_st<F16>(v) : lo_st<F16>(v),
+                                                      j & 1 ? hi_st<F16>(u) : lo_st<F16>(u), acc[q], 0, 0, 0);
+      }
+    // Block 4q + b's sums are registers 4 b .. 4 b + 3: three tree levels.
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float s0 = (acc[0][r] + acc[0][4 + r]) + (acc[0][8 + r] + acc[0][12 + r]);
+      const float s1 = (acc[1][r] + acc[1][4 + r]) + (acc[1][8 + r] + acc[1][12 + r]);
+      sum8[n][r] = s0 + s1;
+    }
+    if (n + 2 < NT)
+      asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    else if (n + 1 < NT)
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+  __syncthreads();  // every wave is done with its rows
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) part[wave][4 * b + r][16 * n + i16] = sum8[n][r];
+  __syncthreads();
+  for (int q = tid; q < 16 * 64; q += 512) {
+    const int t = q >> 6, e = q & 63;
+    if (e < E) {
+      const float lg = ((part[0][t][e] + part[1][t][e]) + (part[2][t][e] + part[3][t][e])) +
+                       ((part[4][t][e] + part[5][t][e]) + (part[6][t][e] + part[7][t][e]));
+      s_logit[t][e] = f2st<F16>(bias ? lg + bias[e] : lg);
+    }
+  }
+  __syncthreads();  // every expert's logits of the block's tokens are in LDS
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+    if (t0 + wave + 8 * k < T)  // wave-uniform
+      rank_token<ROUTE, F16>(s_logit[wave + 8 * k], (int64_t)t0 + wave + 8 * k, E, K, idx, gates_f32, h);
+  __syncthreads();
+  if (tid <= E) hist[(int64_t)blockIdx.x * (E + 1) + tid] = h[tid];
+}
+
+int router_topk_tokens(int T) { return T <= 1024 ? 4 : 16; }
+
+template <int C, int ROUTE, bool F16>
+static void launch_router_topk_c(const uint16_t* x, const uint16_t* w, const float* bias, int T, int H, int E, int K,
+                                 int32_t* idx, float* gates_f32, int32_t* hist, hipStream_t s) {
+  const unsigned tb = (unsigned)router_topk_tokens(T), blocks = ((unsigned)T + tb - 1) / tb;
+#define TFM_RT(kernel) tfm_launch(kernel, blocks, 512, 0, s, x, w, bias, T, H, E, K, idx, gates_f32, hist)
+  if (tb == 4 && E <= 40) TFM_RT((router_topk4_kernel<C, ROUTE, F16, 5>));
+  else if (tb == 4) TFM_RT((router_topk4_kernel<C, ROUTE, F16, 8>));
+  else if (E <= 48) TFM_RT((router_topk16_kernel<C, ROUTE, F16, 3>));
+  else TFM_RT((router_topk16_kernel<C, ROUTE, F16, 4>));
+#undef TFM_RT
+}
+
+template <int C, bool F16>
+static void launch_router_topk_r(int route_kind, const uint16_t* x, const uint16_t* w, const float* bias, int T, int H,
+                                 int E, int K, int32_t* idx, float* gates_f32, int32_t* hist, hipStream_t s) {
+  if (route_kind == TFM_ROUTE_OLMOE)
+    launch_router_topk_c<C, TFM_ROUTE_OLMOE, F16>(x, w, bias, T, H, E, K, idx, gates_f32, hist, s);
+  else
+    launch_router_topk_c<C, TFM_ROUTE_GRANITE, F16>(x, w, bias, T, H, E, K, idx, gates_f32, hist, s);
 }
 
 template <bool F16>
 static bool router_topk_dt(int route_kind, const uint16_t* x, const uint16_t* w, const float* bias,
-                           int T, int H, int E, int K, int32_t* idx, float* gates_f32, int32_t* hist,
-                           uint16_t* logits_out, hipStream_t s) {
+                           int T, int H, int E, int K, int32_t* idx, float* gates_f32, int32_t* hist, hipStream_t s) {
   switch (H) {
-    case 512: launch_router_topk_c<8, F16>(route_kind, x, w, bias, T, H, E, K, idx, gates_f32, hist, logits_out, s); break;
-    case 1024: launch_router_topk_c<16, F16>(route_kind, x, w, bias, T, H, E, K, idx, gates_f32, hist, logits_out, s); break;
-    case 1536: launch_router_topk_c<24, F16>(route_kind, x, w, bias, T, H, E, K, idx, gates_f32, hist, logits_out, s); break;
-    case 2048: launch_router_topk_c<32, F16>(route_kind, x, w, bias, T, H, E, K, idx, gates_f32, hist, logits_out, s); break;
+    case 512: launch_router_topk_r<8, F16>(route_kind, x, w, bias, T, H, E, K, idx, gates_f32, hist, s); break;
+    case 1024: launch_router_topk_r<16, F16>(route_kind, x, w, bias, T, H, E, K, idx, gates_f32, hist, s); break;
+    case 1536: launch_router_topk_r<24, F16>(route_kind, x, w, bias, T, H, E, K, idx, gates_f32, hist, s); break;
+    case 2048: launch_router_topk_r<32, F16>(route_kind, x, w, bias, T, H, E, K, idx, gates_f32, hist, s); break;
     default: return false;
   }
   return true;
 }
 
 bool launch_router_topk(int route_kind, bool f16, const uint16_t* x, const uint16_t* w, const float* bias,
-                        int T, int H, int E, int K, int32_t* idx, float* gates_f32, int32_t* hist,
-                        uint16_t* logits_out, hipStream_t s) {
+                        int T, int H, int E, int K, int32_t* idx, float* gates_f32, int32_t* hist, hipStream_t s) {
   if (T <= 0) return true;
-  const bool ok = f16 ? router_topk_dt<true>(route_kind, x, w, bias, T, H, E, K, idx, gates_f32, hist, logits_out, s)
-                      : router_topk_dt<false>(route_kind, x, w, bias, T, H, E, K, idx, gates_f32, hist, logits_out, s);
+  const bool ok = f16 ? router_topk_dt<true>(route_kind, x, w, bias, T, H, E, K, idx, gates_f32, hist, s)
+                      : router_topk_dt<false>(route_kind, x, w, bias, T, H, E, K, idx, gates_f32, hist, s);
   if (ok) check_hip(hipGetLastError(), "router_topk launch");
   return ok;
 }

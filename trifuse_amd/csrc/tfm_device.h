@@ -153,17 +153,19 @@ __device__ __forceinline__ float row_tree_sum16(float v) {
   return v;
 }
 
-__device__ __forceinline__ float wave_tree_sum64x4(float a, float b, float c, float d) {
-  a = row_tree_sum16(a);
-  b = row_tree_sum16(b);
-  c = row_tree_sum16(c);
-  d = row_tree_sum16(d);
+// The last two levels: a, b, c, d hold one sum per row of 16 lanes; row t
+// returns (row 0 + row 1) + (row 2 + row 3) of value t.
+__device__ __forceinline__ float row_roots4(float a, float b, float c, float d) {
   const auto ab = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
   const auto cd = __builtin_amdgcn_permlane16_swap(__float_as_uint(c), __float_as_uint(d), false, false);
   const float sab = __uint_as_float(ab[0]) + __uint_as_float(ab[1]);  // rows: a01 b01 a23 b23
   const float scd = __uint_as_float(cd[0]) + __uint_as_float(cd[1]);  // rows: c01 d01 c23 d23
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(sab), __float_as_uint(scd), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);               // rows: a b c d
+}
+
+__device__ __forceinline__ float wave_tree_sum64x4(float a, float b, float c, float d) {
+  return row_roots4(row_tree_sum16(a), row_tree_sum16(b), row_tree_sum16(c), row_tree_sum16(d));
 }
 
 __device__ __forceinline__ float silu_mul(float g, float u) {
