@@ -646,28 +646,36 @@ struct Deq8 {
   }
 };
 
-// Tile of BM = 64, 128 or 256 rows. LDS and registers are kept to 48, 80 and
-// 144 KB and 80, 128 and 256 registers, so that three, two and one workgroups
-// share a compute unit: one covers the other's load latency, barriers and
-// epilogue. WV = 4 (64-row tiles only) halves the weight rows of a tile (128:
-// 64 gate and 64 up rows, or 128 down rows) for twice the tiles, where 8-wave
-// tiles would leave compute units idle (a few experts or a few output
-// columns: Granite decode batches, a dense matrix); 40 KB of LDS.
+// Tile of BM = 64, 96, 128 or 256 rows by BN = 16 NJ WV weight rows. Where the
+// LDS and registers allow it, two or more workgroups share a compute unit, and
+// one covers the other's load latency, barriers and epilogue: 64 x 8 waves two
+// (48 KB, 128 registers), 64 x 4 four (40 KB), 96 x 4 (NJ = 4) and 128 x 4 two
+// (64 and 72 KB, 256 registers), 128 x 8 and 256 x 8 one. WV = 4 with NJ = 2
+// halves the weight rows of a tile (128: 64 gate and 64 up rows, or 128 down
+// rows) for twice the tiles, where 8-wave tiles would leave compute units idle
+// (a few experts or a few output columns: Granite decode batches, a dense
+// matrix).
 template <int BM, int WV>
 constexpr int wr_waves_per_simd() { return BM == 64 ? 4 : 2; }
 
-template <int BM, int MODE, int BITS, bool F16, int WV, bool FEW = false>
+template <int BM, int MODE, int BITS, bool F16, int WV, bool FEW = false, int NJ = 2>
 __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM, WV>())) void ggemm_wr_kernel(GgArgs args) {
-  constexpr int WAVES = WV, BN = 32 * WV;
+  constexpr int WAVES = WV, WN = 16 * NJ, BN = WN * WV;
+  constexpr int NB = MODE == kGgGateUp ? NJ / 2 : NJ;  // column blocks of one matrix per wave
   constexpr int MB = BM / 16;                     // 16-row blocks per wave
   constexpr int OUT_COLS = MODE == kGgGateUp ? BN / 2 : BN;
   constexpr int LA = BM / (4 * WAVES);            // 4-row (1 KB) copies per wave per super-step
-  static_assert(WV == 8 || (WV == 4 && BM <= 128), "8 waves, or 4 with 64- and 128-row tiles");
+  static_assert(WV == 8 || (WV == 4 && BM <= 128), "8 waves, or 4 with tiles of up to 128 rows");
+  static_assert(NJ == 2 || (NJ == 4 && WV == 4), "32 weight rows a wave, or 64 with 4 waves");
   static_assert(LA >= 1, "every wave copies activation rows");
   constexpr int SROW = 136;                       // epilogue staging row stride (128 columns + 16 B)
   constexpr int HALF_ROWS = BM / 2;               // staged rows per activation stage
-  static_assert(BM == 64 || BM == 128 || BM == 256, "tile rows");
+  static_assert(BM == 64 || BM == 96 || BM == 128 || BM == 256, "tile rows");
   static_assert(HALF_ROWS * SROW <= BM * BK2, "epilogue staging fits a stage");
+  // 128 rows of 64 weight rows a wave leave no registers for both super-steps'
+  // raw weights: the next one's are requested halfway through sub-step 1, when
+  // half of this one's are used up, and A fragments are read two pairs ahead.
+  constexpr bool LATE = BM == 128 && NJ == 4;
   using op_t = op8_t<F16>;
   using f16tag = std::integral_constant<bool, F16>;
   using D8 = Deq8<BITS, F16>;
@@ -781,21 +789,22 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM, WV>())) void ggemm_
   // ---- weights ----
   const int g4 = lane >> 4;                       // k quarter of the super-step
   const uint32_t qrow = (uint32_t)args.Kin * BITS / 8, srow = (uint32_t)G * 2;
-  __amdgpu_buffer_rsrc_t rbq[2];
-  uint32_t b_qoff[2];
-  int trow[2];                                    // weight row within the tile (0..255)
+  __amdgpu_buffer_rsrc_t rbq[NJ];
+  uint32_t b_qoff[NJ];
+  int trow[NJ];                                   // weight row within the tile (0..255)
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const tfm_affine& bm = (MODE == kGgGateUp && j == 1) ? args.wb : args.wa;
-    trow[j] = MODE == kGgGateUp ? j * (BN / 2) + 16 * wave + (lane & 15) : 32 * wave + 16 * j + (lane & 15);
-    const int bn = MODE == kGgGateUp ? n0 + 16 * wave + (lane & 15) : n0 + 32 * wave + 16 * j + (lane & 15);
+  for (int j = 0; j < NJ; ++j) {
+    const tfm_affine& bm = (MODE == kGgGateUp && j >= NB) ? args.wb : args.wa;
+    const int col = 16 * (NB * wave + j % NB) + (lane & 15);
+    trow[j] = MODE == kGgGateUp ? (j / NB) * (BN / 2) + col : col;
+    const int bn = n0 + col;
     rbq[j] = gg_rsrc(reinterpret_cast<const char*>(bm.q) + (size_t)e * args.N * qrow, (uint32_t)args.N * qrow);
     b_qoff[j] = bn < args.N ? (uint32_t)bn * qrow + 4u * BITS * g4 : kOob;
   }
   auto bload = [&](uint4 (*raw)[RL], int kt) {
     const bool live = kt < KT;
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < NJ; ++j)
 #pragma unroll
       for (int r = 0; r < RL; ++r)
         raw[j][r] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(live ? rbq[j] : rnull, b_qoff[j] + 16 * r, kt * 16 * BITS, 0));
@@ -810,24 +819,30 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM, WV>())) void ggemm_
   // Loaded straight into registers instead, as 2-byte values of 64 rows at a
   // time, they cost as much as the packed codes; kept for the whole input
   // width (32 KB at 2048) they cost 128-row tiles a workgroup per compute unit.
-  const int sw = wave % (WAVES / 2);              // rows 64 sw .. 64 sw + 63 of the tile
-  const bool sbias = wave >= WAVES / 2, sup = MODE == kGgGateUp && 64 * sw >= BN / 2;
-  const tfm_affine& sm = sup ? args.wb : args.wa;
-  const auto rsb = gg_rsrc(static_cast<const char*>(sbias ? sm.biases : sm.scales) + (size_t)e * args.N * srow,
-                           (uint32_t)args.N * srow);
-  const int sn0 = n0 + 64 * sw - (sup ? BN / 2 : 0);  // matrix row of the first
+  // Piece p of 2 BN / 64: scales (p < BN / 64) or biases of rows 64 sw .. + 63.
+  constexpr int SBP = 2 * BN / (64 * WAVES);      // pieces per wave
   const bool sb16 = (G & 7) == 0;
   auto sb_copy = [&](int c) {
-    uint16_t* const dst = sSb + ((c & 1) * 2 + (sbias ? 1 : 0)) * SBH + 64 * 8 * sw;
-    const bool live = 8 * c < G;
-    if (sb16) {
-      const int n = sn0 + lane;
-      lds_dma16(rsb, dst, live && n < args.N ? (uint32_t)n * srow + 16u * c : kOob, 0);
-    } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {               // dword 64 i + lane: row 16 i + lane / 4, pair lane % 4
-        const int n = sn0 + 16 * i + (lane >> 2);
-        lds_dma4(rsb, dst + 128 * i, live && n < args.N ? (uint32_t)n * srow + 16u * c + 4u * (lane & 3) : kOob);
+    for (int u = 0; u < SBP; ++u) {
+      const int p = u * WAVES + wave;
+      const int sw = p % (BN / 64);
+      const bool sbias = p >= BN / 64, sup = MODE == kGgGateUp && 64 * sw >= BN / 2;
+      const tfm_affine& sm = sup ? args.wb : args.wa;
+      const auto rsb = gg_rsrc(static_cast<const char*>(sbias ? sm.biases : sm.scales) + (size_t)e * args.N * srow,
+                               (uint32_t)args.N * srow);
+      const int sn0 = n0 + 64 * sw - (sup ? BN / 2 : 0);  // matrix row of the first
+      uint16_t* const dst = sSb + ((c & 1) * 2 + (sbias ? 1 : 0)) * SBH + 64 * 8 * sw;
+      const bool live = 8 * c < G;
+      if (sb16) {
+        const int n = sn0 + lane;
+        lds_dma16(rsb, dst, live && n < args.N ? (uint32_t)n * srow + 16u * c : kOob, 0);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {             // dword 64 i + lane: row 16 i + lane / 4, pair lane % 4
+          const int n = sn0 + 16 * i + (lane >> 2);
+          lds_dma4(rsb, dst + 128 * i, live && n < args.N ? (uint32_t)n * srow + 16u * c + 4u * (lane & 3) : kOob);
+        }
       }
     }
   };
@@ -837,14 +852,14 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM, WV>())) void ggemm_
     g = g < G ? g : G - 1;
     const uint16_t* const p = sSb + ((g >> 3) & 1) * 2 * SBH + (g & 7);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < NJ; ++j) {
       sc[j] = D8::sb(p[trow[j] * 8]);
       bi[j] = D8::sb(p[trow[j] * 8 + SBH]);
     }
   };
   auto deq = [&](op_t* b, uint4 (*raw)[RL], const sb_t* sc, const sb_t* bi) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < NJ; ++j) {
       D8 d;
       uint32_t o[4];
       const uint32_t* w = reinterpret_cast<const uint32_t*>(&raw[j][0]);
@@ -853,11 +868,11 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM, WV>())) void ggemm_
     }
   };
 
-  f32x4_t acc[MB][2];
+  f32x4_t acc[MB][NJ];
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
   // One super-step on activation stage A: sub-step s runs the MFMAs of the
   // MBL live row blocks with B operand b (word s) and dequantises the B
@@ -878,16 +893,16 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM, WV>())) void ggemm_
   const uint32_t a_lane = (uint32_t)((lane & 15) * BK2 * 2 + (((4 * g4) ^ (lane & 15)) << 4));
   auto compute = [&](auto mbl_tag, const uint16_t* A, op_t* b, uint4 (*rc)[RL], const sb_t* sc,
                      const sb_t* bic, uint4 (*rn)[RL], const sb_t* sn, const sb_t* bin, uint16_t* An,
-                     int ktn, auto after_copy) __attribute__((always_inline)) {
+                     int ktn, auto weight_load) __attribute__((always_inline)) {
     constexpr int MBL = decltype(mbl_tag)::value;
-    constexpr int NQ = 4 * MBL, D = 3, R = D + 1;
+    constexpr int NQ = 4 * MBL, D = LATE ? 2 : 3, R = D + 1;
     constexpr int CR = 4 * WAVES;  // rows per copy round
     constexpr int NC = (16 * MBL + CR - 1) / CR < LA ? (16 * MBL + CR - 1) / CR : LA;
     constexpr int STEP = NQ / (2 * NC) > 0 ? NQ / (2 * NC) : 1;
     static_assert(STEP * (NC - 1) < NQ, "every copy is issued");
     op_t af[R];
-    uint32_t nbw[2][4];                           // next B operand, packed pairs
-    D8 dq[2];
+    uint32_t nbw[NJ][4];                          // next B operand, packed pairs
+    D8 dq[NJ];
     uint32_t al = a_lane;
     asm volatile("" : "+v"(al));
     const char* const Ab = reinterpret_cast<const char*>(A);
@@ -900,14 +915,14 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM, WV>())) void ggemm_
     static_for<0, NQ>([&](auto q_) {
       constexpr int q = decltype(q_)::value, s = q / MBL, i = q % MBL;
       if constexpr (q % STEP == 0 && q / STEP < NC) a_copy1(An, ktn, std::integral_constant<int, q / STEP>{});
-      if constexpr (q == STEP * (NC - 1)) after_copy();
+      if constexpr (q == (LATE ? MBL + MBL / 2 : STEP * (NC - 1))) weight_load();
       if constexpr (q + D < NQ) rd(std::integral_constant<int, q + D>{});
-      acc[i][0] = mfma16(af[q % R], b[0], acc[i][0], f16tag{});
-      acc[i][1] = mfma16(af[q % R], b[1], acc[i][1], f16tag{});
-      // Slices of the next sub-step's B operand: slice c of 16 is slice c % 8
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) acc[i][j] = mfma16(af[q % R], b[j], acc[i][j], f16tag{});
+      // Slices of the next sub-step's B operand: slice c of 8 NJ is slice c % 8
       // of row c / 8 (word(s) s + 1, or the first of the next super-step's raw
       // weights).
-      constexpr int c0 = 16 * i / MBL, c1 = 16 * (i + 1) / MBL;
+      constexpr int c0 = 8 * NJ * i / MBL, c1 = 8 * NJ * (i + 1) / MBL;
       static_for<c0, c1>([&](auto c_) {
         constexpr int c = decltype(c_)::value, j = c / 8, el = c % 8;
         constexpr int w0 = s < 3 ? RL * (s + 1) : 0;
@@ -916,7 +931,7 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM, WV>())) void ggemm_
       });
       if constexpr (i == MBL - 1) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < NJ; ++j)
           b[j] = __builtin_bit_cast(op_t, make_uint4(nbw[j][0], nbw[j][1], nbw[j][2], nbw[j][3]));
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -947,6 +962,11 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM, WV>())) void ggemm_
       else if (rows_valid > 64) f(std::integral_constant<int, 6>{});
       else if (rows_valid > 32) f(std::integral_constant<int, 4>{});
       else f(std::integral_constant<int, 2>{});
+    } else if constexpr (MB == 6) {
+      if (rows_valid > 80) f(std::integral_constant<int, 6>{});
+      else if (rows_valid > 64) f(std::integral_constant<int, 5>{});
+      else if (rows_valid > 32) f(std::integral_constant<int, 4>{});
+      else f(std::integral_constant<int, 2>{});
     } else {
       if (rows_valid > 32) f(std::integral_constant<int, 4>{});
       else if (rows_valid > 16) f(std::integral_constant<int, 2>{});
@@ -956,9 +976,9 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM, WV>())) void ggemm_
   constexpr bool AHEAD = FEW;
   if (AHEAD && (BM == 128 || rows_valid <= 16) && (KT & 3) == 0) {
     if constexpr (AHEAD) {
-      uint4 rw[4][2][RL];                         // raw weights of super-step k in slot k % 4
-      sb_t fsc[2][2], fbi[2][2];                  // scales and biases of super-step k in set k % 2
-      op_t fb[2];
+      uint4 rw[4][NJ][RL];                         // raw weights of super-step k in slot k % 4
+      sb_t fsc[2][NJ], fbi[2][NJ];                  // scales and biases of super-step k in set k % 2
+      op_t fb[NJ];
       sb_copy(0);
       a_copy(sA0, 0);
       bload(rw[0], 0);
@@ -992,9 +1012,9 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM, WV>())) void ggemm_
     }
   } else {
   // ---- prologue ----
-  uint4 r0[2][RL], r1[2][RL];
-  sb_t sc0[2], bi0[2], sc1[2], bi1[2];
-  op_t bop[2];
+  uint4 r0[NJ][RL], r1[NJ][RL];
+  sb_t sc0[NJ], bi0[NJ], sc1[NJ], bi1[NJ];
+  op_t bop[NJ];
   sb_copy(0);
   a_copy(sA0, 0);
   bload(r0, 0);
@@ -1010,16 +1030,16 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM, WV>())) void ggemm_
   // its first read comes in super-step 4c + 3.
   auto main_loop = [&](auto mbl_tag) {
     for (int kt = 0; kt < KT; kt += 2) {
-      bload(r1, kt + 1);
+      if constexpr (!LATE) bload(r1, kt + 1);
       sb_read(sc1, bi1, kt + 1);
       if ((kt & 3) == 0) sb_copy(kt / 4 + 1);
       __builtin_amdgcn_sched_barrier(0);
-      compute(mbl_tag, sA0, bop, r0, sc0, bi0, r1, sc1, bi1, sA1, kt + 1, [] {});
+      compute(mbl_tag, sA0, bop, r0, sc0, bi0, r1, sc1, bi1, sA1, kt + 1, [&] { if constexpr (LATE) bload(r1, kt + 1); });
       __syncthreads();
-      bload(r0, kt + 2);
+      if constexpr (!LATE) bload(r0, kt + 2);
       sb_read(sc0, bi0, kt + 2);
       __builtin_amdgcn_sched_barrier(0);
-      compute(mbl_tag, sA1, bop, r1, sc1, bi1, r0, sc0, bi0, sA0, kt + 2, [] {});
+      compute(mbl_tag, sA1, bop, r1, sc1, bi1, r0, sc0, bi0, sA0, kt + 2, [&] { if constexpr (LATE) bload(r0, kt + 2); });
       __syncthreads();
     }
   };
@@ -1040,7 +1060,7 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM, WV>())) void ggemm_
   static_for<0, PASSES>([&](auto p_) {
     constexpr int p = decltype(p_)::value;
     if (p > 0) __syncthreads();  // the previous pass's reads are done
-    const bool mine = MODE == kGgGateUp || (wave >> 2) == p;
+    const bool mine = MODE == kGgGateUp || WN * wave / 128 == p;
     if (mine) {
       static_for<0, MB>([&](auto i_) {
         constexpr int i = decltype(i_)::value;
@@ -1050,10 +1070,12 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM, WV>())) void ggemm_
           const int row = 16 * i + 4 * g4 + v;
           uint16_t* st = (row < HALF_ROWS ? sA0 : sA1) + (row % HALF_ROWS) * SROW;
           if constexpr (MODE == kGgGateUp) {
-            st[16 * wave + (lane & 15)] = f2st<F16>(swiglu(acc[i][0][v], acc[i][1][v]));
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+              st[16 * (NB * wave + j) + (lane & 15)] = f2st<F16>(swiglu(acc[i][j][v], acc[i][j + NB][v]));
           } else {
 #pragma unroll
-            for (int j = 0; j < 2; ++j) st[32 * (wave & 3) + 16 * j + (lane & 15)] = f2st<F16>(acc[i][j][v]);
+            for (int j = 0; j < NJ; ++j) st[WN * wave % 128 + 16 * j + (lane & 15)] = f2st<F16>(acc[i][j][v]);
           }
         }
       });
@@ -1087,7 +1109,7 @@ static int down_tile_override() {
   static int v = [] {
     const char* s = std::getenv("TFM_GGEMM_DOWN_TILE");
     const int n = s ? std::atoi(s) : 0;
-    return n == 64 || n == 128 || n == 256 ? n : 0;
+    return n == 64 || n == 96 || n == 128 || n == 256 ? n : 0;
   }();
   return v;
 }
@@ -1120,9 +1142,10 @@ static int gg_device_cus() {
   return cus;
 }
 
-// Tile of the weights-in-registers kernel: rows BM and waves WV.
+// Tile of the weights-in-registers kernel: rows BM, waves WV and 16-row weight
+// blocks a wave NJ.
 struct WrTile {
-  int bm, wv;
+  int bm, wv, nj;
 };
 
 // Chosen from the average routes per expert a = n_routes / E and the number
@@ -1133,6 +1156,14 @@ struct WrTile {
 //  * A dense matrix (few experts and columns): the largest tile whose count
 //    fills the compute units, else 64 x 4 (2048 x 2048 linear: 1024 rows 64x4
 //    19.1, 128x4 23.7; 2048 rows 28.4 and 26.4).
+//  * 96 x 4 (64 weight rows a wave: half the LDS reads and activation copies
+//    per product), 4-bit codes, wide, where experts of about a routes fill one
+//    such tile (44 < a <= 72, three deviations of evenly spread routes below
+//    96) or two where 128 rows would take two as well (128 < a <= 155). us per
+//    layer, gate/up and down, against the other tiles: OLMoE 400 tokens 106.8
+//    and 114.4, 512 tokens 118.5 and 125.0, 1111 tokens 193.3 and 203.7; past
+//    the fit it loses: 700 tokens 162.5 and 136.1, 900 tokens 183.9 and 170.2.
+//    Not 8-bit codes, whose raw weights leave it too few registers.
 //  * Down. 64 x 4 up to a = 44 (OLMoE 300 tokens, a = 38: 29.2 against 32.8 on
 //    128x4; 400 tokens: 34.7 and 34.2), then 128 x 4 (512 tokens 38.2 against
 //    42.0 on 64x4 and 40.0 on 128x8; Granite 1024 tokens 27.6, 28.3 on 256x8;
@@ -1155,35 +1186,57 @@ struct WrTile {
 //    an expert has one m-tile (512 tokens 61.7 against 64.4 on 128x4; half
 //    58.0 and 62.6), four above (900 tokens 97.4 against 102.2; Granite 2048
 //    71.8 and 78.3).
-// TFM_GGEMM_TILE=64/128/256 forces the rows, TFM_GGEMM_DOWN_TILE those of the
+//  * Gate/up of 4-bit codes with bf16 storage: 128 x 4 with 64 weight rows a
+//    wave, against the tile above: wide 700 tokens (a = 87) 66.9 and 71.6, 800
+//    tokens 78.0 and 75.8, 1000 tokens 104.0 and 106.5, 1300 tokens 120.6 and
+//    131.6, 1750 tokens 130.2 and 144.0, 2400 tokens 178.3 and 187.7, 4000
+//    tokens 277.0 and 271.6 (256x8). Not wide, where its rounds are full
+//    enough: Granite 1024 tokens (a = 205, 336 tiles in a round of 512) 47.8
+//    and 43.4, 1500 tokens (454) 51.2 and 54.5, 2048 tokens (592 in two) 10 us
+//    a layer slower, 2500 tokens (704) 74.6 and 84.5, 4000 tokens (1080 in
+//    three) 114.9 and 123.9. (The down GEMM is level or slower on it; half storage
+//    has too few registers for it.)
+// TFM_GGEMM_TILE=64/96/128/256 forces the rows, TFM_GGEMM_DOWN_TILE those of the
 // down GEMM alone (TFM_GGEMM_TILE takes precedence), TFM_GGEMM_WAVES=4/8 the
 // waves.
-static WrTile wr_tile(int64_t n_routes, int E, int64_t cols, int kin, int mode, int bits) {
+static WrTile wr_tile(int64_t n_routes, int E, int64_t cols, int kin, int mode, int bits, bool f16) {
   const int64_t cus = gg_device_cus();
   auto mtiles = [&](int bm) { return (n_routes + (int64_t)E * bm - 1) / ((int64_t)E * bm); };
+  auto upto = [&](int a) { return n_routes <= (int64_t)E * a; };  // average routes at most a
   auto pick = [&]() -> WrTile {
     if (4 * E * cols < cus) {
-      if (E * mtiles(256) * cols >= cus) return {256, 8};
-      if (E * mtiles(128) * cols * 2 >= cus) return {128, 4};
-      return {64, 4};
+      if (E * mtiles(256) * cols >= cus) return {256, 8, 2};
+      if (E * mtiles(128) * cols * 2 >= cus) return {128, 4, 2};
+      return {64, 4, 2};
     }
     const bool wide = E * cols >= cus;
+    if (wide && bits == 4 && ((!upto(44) && upto(72)) || (!upto(128) && upto(155)))) return {96, 4, 4};
     if (mode == kGgDown) {
-      if (n_routes <= (int64_t)E * (bits == 8 ? 56 : 44)) return {64, 4};
-      if (n_routes >= (int64_t)E * 448 && kin >= 1024) return {256, 8};
-      return {128, 4};
+      if (upto(bits == 8 ? 56 : 44)) return {64, 4, 2};
+      if (n_routes >= (int64_t)E * 448 && kin >= 1024) return {256, 8, 2};
+      return {128, 4, 2};
     }
-    if (n_routes <= (int64_t)E * (wide && bits == 4 ? 44 : 56))
-      return {64, n_routes > 2 * E && E * mtiles(64) * cols >= 2 * cus ? 8 : 4};
-    if (n_routes >= (int64_t)E * (wide ? 232 : 480)) return {256, 8};
-    return {128, n_routes <= (int64_t)E * 104 ? 8 : 4};
+    if (upto(wide && bits == 4 ? 44 : 56))
+      return {64, n_routes > 2 * E && E * mtiles(64) * cols >= 2 * cus ? 8 : 4, 2};
+    if (mode == kGgGateUp && bits == 4 && !f16) {
+      if (wide && (upto(96) || (!upto(112) && upto(400)))) return {128, 4, 4};
+      // Tiles of E experts of a / 128 + 1/2 m-tiles, two a compute unit: the
+      // rounds must be two thirds full.
+      const int64_t tiles = (n_routes + (int64_t)E * 64) * cols / 128, round = 2 * cus;
+      if (!wide && !upto(150) && 3 * tiles >= 2 * ((tiles + round - 1) / round) * round) return {128, 4, 4};
+    }
+    if (n_routes >= (int64_t)E * (wide ? 232 : 480)) return {256, 8, 2};
+    return {128, upto(104) ? 8 : 4, 2};
   };
-  WrTile t = pick();
+  const WrTile t = pick();
   int bm = tile_override();
-  if (bm != 64 && bm != 128 && bm != 256) bm = mode == kGgDown ? down_tile_override() : 0;
-  if (bm && bm != t.bm) t = {bm, bm == 64 ? 4 : 8};
-  if (waves_override() && t.bm != 256) t.wv = waves_override();
-  return t;
+  if (bm != 64 && bm != 96 && bm != 128 && bm != 256) bm = mode == kGgDown ? down_tile_override() : 0;
+  const int wv = waves_override();
+  if (!bm && !wv) return t;
+  if (!bm) bm = t.bm;
+  if (bm == 96) return {96, 4, 4};
+  if (bm == 256) return {256, 8, 2};
+  return {bm, wv ? wv : bm == t.bm ? t.wv : bm == 64 ? 4 : 8, 2};
 }
 
 static unsigned grid_for(int64_t n_routes, int E, int BM, int NT) {
@@ -1218,9 +1271,9 @@ static bool use_few_rows(int64_t n_routes, int E) {
   return v == 2 || (v == 1 && n_routes <= (int64_t)E * kFewRowsAvg);
 }
 
-template <int BM, int MODE, int BITS, bool F16, int WV>
+template <int BM, int MODE, int BITS, bool F16, int WV, int NJ = 2>
 static void launch_wr(const GgArgs& a, int64_t n_routes, int E, hipStream_t s) {
-  constexpr int OUT_COLS = MODE == kGgGateUp ? 16 * WV : 32 * WV;
+  constexpr int OUT_COLS = (MODE == kGgGateUp ? 8 : 16) * NJ * WV;
   const int NT = (a.N + OUT_COLS - 1) / OUT_COLS;
   // With 256-row tiles an XCD's run of cheap tiles holds more tiles than an
   // even share: at most share x 29 / 17 + 2 (full tile 29 units, cheapest
@@ -1233,7 +1286,7 @@ static void launch_wr(const GgArgs& a, int64_t n_routes, int E, hipStream_t s) {
       return;
     }
   }
-  tfm_launch(ggemm_wr_kernel<BM, MODE, BITS, F16, WV>, grid, WV * 64, 0, s, a);
+  tfm_launch(ggemm_wr_kernel<BM, MODE, BITS, F16, WV, false, NJ>, grid, WV * 64, 0, s, a);
 }
 
 // Inputs a multiple of 128 wide: weights in registers (ggemm_wr_kernel);
@@ -1242,7 +1295,19 @@ template <int MODE, int BITS, bool F16>
 static void launch_tile(const GgArgs& a, int64_t n_routes, int E, hipStream_t s) {
   if (a.Kin % BK2 == 0) {
     const WrTile t = wr_tile(n_routes, E, MODE == kGgGateUp ? (2 * (int64_t)a.N + 255) / 256 : ((int64_t)a.N + 255) / 256,
-                             a.Kin, MODE, BITS);
+                             a.Kin, MODE, BITS, F16);
+    if constexpr (BITS == 4) {
+      if (t.bm == 96) {
+        launch_wr<96, MODE, BITS, F16, 4, 4>(a, n_routes, E, s);
+        return;
+      }
+    }
+    if constexpr (BITS == 4 && !F16 && MODE == kGgGateUp) {
+      if (t.bm == 128 && t.nj == 4) {
+        launch_wr<128, MODE, BITS, F16, 4, 4>(a, n_routes, E, s);
+        return;
+      }
+    }
     if (t.bm == 256) launch_wr<256, MODE, BITS, F16, 8>(a, n_routes, E, s);
     else if (t.bm == 128 && t.wv == 8) launch_wr<128, MODE, BITS, F16, 8>(a, n_routes, E, s);
     else if (t.bm == 128) launch_wr<128, MODE, BITS, F16, 4>(a, n_routes, E, s);
