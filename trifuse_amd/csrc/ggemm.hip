@@ -1,5 +1,9 @@
 // Prefill path: grouped GEMM over expert-contiguous routes.
 //
+// Two kernels: ggemm_wr_kernel (weights in registers; input widths a multiple
+// of 128, described below at its definition) and ggemm_kernel, for odd
+// multiples of 64:
+//
 // Each workgroup computes a BM x BN tile of one expert's output with eight
 // waves, two per SIMD, so that one wave's loads, dequantisation and LDS
 // traffic overlap the other's MFMAs. Per K step of 64 (one quantisation
@@ -655,11 +659,11 @@ struct Deq8 {
 // rows) for twice the tiles, where 8-wave tiles would leave compute units idle
 // (a few experts or a few output columns: Granite decode batches, a dense
 // matrix).
-template <int BM, int WV>
+template <int BM>
 constexpr int wr_waves_per_simd() { return BM == 64 ? 4 : 2; }
 
 template <int BM, int MODE, int BITS, bool F16, int WV, bool FEW = false, int NJ = 2>
-__global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM, WV>())) void ggemm_wr_kernel(GgArgs args) {
+__global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM>())) void ggemm_wr_kernel(GgArgs args) {
   constexpr int WAVES = WV, WN = 16 * NJ, BN = WN * WV;
   constexpr int NB = MODE == kGgGateUp ? NJ / 2 : NJ;  // column blocks of one matrix per wave
   constexpr int MB = BM / 16;                     // 16-row blocks per wave
@@ -949,8 +953,9 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM, WV>())) void ggemm_
   // only for that copy (the vector memory counter retires in issue order), so
   // they stay in flight across it. The products and their order are those of
   // the loop below.
-  // Live row blocks (uniform over the workgroup): in steps of four of 16
-  // blocks, of two of 8; with 64-row tiles 1, 2 or 4 (16, 32 or 64 rows).
+  // Live row blocks (uniform over the workgroup), so that empty rows cost no
+  // MFMAs: in steps of four of 16 blocks, of two of 8; 2, 4, 5 or 6 with 96-row
+  // tiles; 1, 2 or 4 with 64-row ones (16, 32 or 64 rows).
   auto by_live = [&](auto f) __attribute__((always_inline)) {
     if constexpr (MB == 16) {
       if (rows_valid > 192) f(std::integral_constant<int, 16>{});
@@ -973,9 +978,9 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM, WV>())) void ggemm_
       else f(std::integral_constant<int, 1>{});
     }
   };
-  constexpr bool AHEAD = FEW;
-  if (AHEAD && (BM == 128 || rows_valid <= 16) && (KT & 3) == 0) {
-    if constexpr (AHEAD) {
+  if (FEW && rows_valid <= 16 && (KT & 3) == 0) {
+    if constexpr (FEW) {
+      static_assert(BM == 64, "few-row tiles are 64-row tiles");
       uint4 rw[4][NJ][RL];                         // raw weights of super-step k in slot k % 4
       sb_t fsc[2][NJ], fbi[2][NJ];                  // scales and biases of super-step k in set k % 2
       op_t fb[NJ];
@@ -986,7 +991,6 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM, WV>())) void ggemm_
       __syncthreads();  // scale copies and stage 0 complete and visible
       sb_read(fsc[0], fbi[0], 0);
       deq(fb, rw[0], fsc[0], fbi[0]);
-      auto ahead_loop = [&](auto mbl_tag) __attribute__((always_inline)) {
       for (int kt0 = 0; kt0 < KT; kt0 += 4) {
         static_for<0, 4>([&](auto q_) {
           constexpr int q = decltype(q_)::value, c = q % 2, n = 1 - c;
@@ -996,7 +1000,7 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM, WV>())) void ggemm_
           sb_read(fsc[n], fbi[n], kt + 1);
           if constexpr (q == 0) sb_copy(kt0 / 4 + 1);
           __builtin_amdgcn_sched_barrier(0);
-          compute(mbl_tag, A, fb, rw[q], fsc[c], fbi[c], rw[(q + 1) % 4], fsc[n],
+          compute(std::integral_constant<int, 1>{}, A, fb, rw[q], fsc[c], fbi[c], rw[(q + 1) % 4], fsc[n],
                   fbi[n], An, kt + 1, [&] { bload(rw[(q + 2) % 4], kt + 2); });
           // This wave's copies are done (only the 2 RL weight loads issued
           // after them may be outstanding), then every wave's.
@@ -1006,9 +1010,6 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM, WV>())) void ggemm_
             asm volatile("s_waitcnt vmcnt(4)\n\ts_barrier" ::: "memory");
         });
       }
-      };
-      if constexpr (FEW) ahead_loop(std::integral_constant<int, 1>{});
-      else by_live(ahead_loop);
     }
   } else {
   // ---- prologue ----
