@@ -1226,6 +1226,10 @@ static WrTile wr_tile(int64_t n_routes, int E, int64_t cols, int kin, int mode, 
       const int64_t tiles = (n_routes + (int64_t)E * 64) * cols / 128, round = 2 * cus;
       if (!wide && !upto(150) && 3 * tiles >= 2 * ((tiles + round - 1) / round) * round) return {128, 4, 4};
     }
+    // 256-row tiles in one round of the compute units where 128-row ones need
+    // more (Granite 700 tokens, a = 140: 35.1 against 38.8 on 128x4; 8-bit codes
+    // 1000 tokens 45.5 and 49.6).
+    if (!wide && E * mtiles(128) * cols > cus && E * mtiles(256) * cols <= cus) return {256, 8, 2};
     if (n_routes >= (int64_t)E * (wide ? 232 : 480)) return {256, 8, 2};
     return {128, upto(104) ? 8 : 4, 2};
   };
