@@ -12,6 +12,11 @@ from trifuse_amd import workload as wl
 pytestmark = pytest.mark.gpu
 
 DT = {"bf16": torch.bfloat16, "f16": torch.float16}
+# A product's largest error over its largest value. A weight and the result
+# are each rounded to the storage type (half a step: 2^-9 of a bf16 value, 2^-12
+# of a half one). Weight errors add up as a random walk and stay below half a
+# step of the largest result; the fp32 sums add 1e-6. Twice the half step.
+STEP = {"bf16": 2.0 ** -8, "f16": 2.0 ** -11}
 
 
 def _affine(shape, bits, dtype, key, device):
@@ -84,6 +89,40 @@ def test_product_shapes(gpu, dtype, bits, E, N, Kin, rows):
     err = max_rel(oracle.st_to_f32(u16(out)[pick], dtype), ref)
     log(f"  max_rel {err:.2e}")
     assert err <= BLOCK_TOL
+
+
+def _shifted(t, elements):
+    """t's values in an array that starts `elements` 2-byte elements past an aligned one."""
+    buf = torch.zeros(t.numel() + elements, dtype=t.dtype, device=t.device)
+    out = buf[elements:].view(t.shape)
+    out.copy_(t)
+    assert out.is_contiguous() and out.data_ptr() % 16 == (2 * elements) % 16
+    return out
+
+
+# Scales and biases that start at any element of an allocation: 2-byte
+# boundaries (the LDS-dequantising kernel's 2-byte loads), 4-byte ones (dword
+# copies) and 16-byte ones, on both sides of 2048 and at odd multiples of 64.
+# Dword and 16-byte copies move the same values: the same bits.
+@pytest.mark.parametrize("dtype,bits", [("bf16", 4), ("f16", 4), ("bf16", 8), ("f16", 8)])
+@pytest.mark.parametrize("Kin", [192, 512, 2304, 3072])
+def test_scale_alignment(gpu, dtype, bits, Kin):
+    E, N, rows = 3, 128, 300
+    q, s, b = _affine((E, N, Kin), bits, dtype, 11 * Kin + bits, gpu)
+    x = wl.normal_bf16((rows, Kin), 1.0, Kin, dtype=DT[dtype])
+    rhs = np.random.default_rng(Kin).integers(0, E, size=rows).astype(np.int32)
+    ref = oracle.gather_qmm_f64(u16(x), np.arange(rows), rhs, u32(q), u16(s), u16(b), dtype=dtype)
+    got = {}
+    for shift in ((0, 0), (1, 1), (2, 2), (0, 1), (3, 0), (8, 2)):
+        log(f"alignment {dtype} bits={bits} Kin={Kin} scales +{shift[0]} biases +{shift[1]}")
+        out = tmoe.gather_qmm_rows(x.to(gpu), q, _shifted(s, shift[0]), _shifted(b, shift[1]),
+                                   torch.from_numpy(rhs).to(gpu), bits=bits)
+        torch.cuda.synchronize()
+        got[shift] = u16(out)
+        err = max_rel(oracle.st_to_f32(got[shift], dtype), ref)
+        assert err <= STEP[dtype], (shift, err)
+    for shift in ((2, 2), (8, 2)):
+        np.testing.assert_array_equal(got[shift], got[0, 0])
 
 
 # Around the router kernels' switches (64 and 1024 tokens), token counts off 4

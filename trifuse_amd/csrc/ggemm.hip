@@ -14,7 +14,8 @@
 //   * loads BN packed weight rows (4-bit: 32 bytes, 8-bit: 64 bytes of each
 //     row per step) into registers, dequantises them (s*q+b in fp32,
 //     rounded to the storage dtype, bf16 or half) and writes them to LDS;
-//     for inputs up to 2048 wide the scales and biases of the tile's rows
+//     for inputs up to 2048 wide (and arrays on 16-byte boundaries) the scales
+//     and biases of the tile's rows
 //     are copied into LDS once per tile (coalesced) instead of being loaded
 //     per step as 2-byte values from 64 rows at a time,
 //   * runs v_mfma_f32_32x32x16_bf16 (or _f16) on the two LDS tiles, each wave owning a
@@ -72,6 +73,7 @@ struct GgArgs {
   int N;                 // output columns of one matrix
   int Kin;
   uint16_t* out;         // gate/up: h [n_routes, N]; down: y [n_routes, N]; plain: out [rows, N]
+  int sb16;              // ggemm_wr_kernel: scale and bias rows start on 16-byte boundaries
 };
 
 // Row of accumulator element v of lane `lane` inside a 32x32 block of
@@ -817,15 +819,16 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM>())) void ggemm_wr_k
   // Scales and biases: chunk c holds groups 8c..8c+7 (super-steps 4c..4c+3) of
   // the tile's BN rows, 16 bytes a row, in ring slot c % 2. The first half of
   // the waves copies scales, the second biases, 64 rows each: one 16-byte
-  // LDS-DMA per wave and chunk. Rows of G groups not a multiple of 8 are only
-  // 4-byte aligned and take four 4-byte copies. A row's last chunk may read
+  // LDS-DMA per wave and chunk. Rows that start on 4-byte boundaries only (G
+  // not a multiple of 8, or arrays off a 16-byte boundary) take four 4-byte
+  // copies. A row's last chunk may read
   // past its groups (the next row's, never used, or zeros past the matrix).
   // Loaded straight into registers instead, as 2-byte values of 64 rows at a
   // time, they cost as much as the packed codes; kept for the whole input
   // width (32 KB at 2048) they cost 128-row tiles a workgroup per compute unit.
   // Piece p of 2 BN / 64: scales (p < BN / 64) or biases of rows 64 sw .. + 63.
   constexpr int SBP = 2 * BN / (64 * WAVES);      // pieces per wave
-  const bool sb16 = (G & 7) == 0;
+  const bool sb16 = args.sb16 != 0;
   auto sb_copy = [&](int c) {
 #pragma unroll
     for (int u = 0; u < SBP; ++u) {
@@ -1253,11 +1256,18 @@ static unsigned grid_for(int64_t n_routes, int E, int BM, int NT) {
   return (unsigned)total;
 }
 
+// Low address bits of the scale and bias arrays, which a caller may start at
+// any element: copies into LDS need 4- or 16-byte boundaries.
+static uintptr_t sb_address_bits(const GgArgs& a) {
+  return reinterpret_cast<uintptr_t>(a.wa.scales) | reinterpret_cast<uintptr_t>(a.wa.biases) |
+         reinterpret_cast<uintptr_t>(a.wb.scales) | reinterpret_cast<uintptr_t>(a.wb.biases);
+}
+
 template <int BM_, int BN_, int WAVES_M, int WAVES_N, int MODE, int BITS, bool F16>
 static void launch_one(const GgArgs& a, int64_t n_routes, int E, hipStream_t s) {
   using C = GgCfg<BM_, BN_, WAVES_M, WAVES_N, MODE, BITS>;
   const int NT = (a.N + C::OUT_COLS - 1) / C::OUT_COLS;
-  if (a.Kin <= kLdsScaleKin)
+  if (a.Kin <= kLdsScaleKin && (sb_address_bits(a) & 15) == 0)
     tfm_launch(ggemm_kernel<BM_, BN_, WAVES_M, WAVES_N, MODE, BITS, F16, true>, grid_for(n_routes, E, BM_, NT), C::THREADS, 0, s, a);
   else
     tfm_launch(ggemm_kernel<BM_, BN_, WAVES_M, WAVES_N, MODE, BITS, F16, false>, grid_for(n_routes, E, BM_, NT), C::THREADS, 0, s, a);
@@ -1295,10 +1305,14 @@ static void launch_wr(const GgArgs& a, int64_t n_routes, int E, hipStream_t s) {
 }
 
 // Inputs a multiple of 128 wide: weights in registers (ggemm_wr_kernel);
-// otherwise (odd multiples of 64) ggemm_kernel.
+// otherwise (odd multiples of 64, or scales or biases off a 4-byte boundary,
+// which only 2-byte loads reach) ggemm_kernel.
 template <int MODE, int BITS, bool F16>
-static void launch_tile(const GgArgs& a, int64_t n_routes, int E, hipStream_t s) {
-  if (a.Kin % BK2 == 0) {
+static void launch_tile(const GgArgs& a_in, int64_t n_routes, int E, hipStream_t s) {
+  GgArgs a = a_in;
+  const uintptr_t sb = sb_address_bits(a);
+  a.sb16 = (sb & 15) == 0 && a.Kin / BK % 8 == 0;
+  if (a.Kin % BK2 == 0 && (sb & 3) == 0) {
     const WrTile t = wr_tile(n_routes, E, MODE == kGgGateUp ? (2 * (int64_t)a.N + 255) / 256 : ((int64_t)a.N + 255) / 256,
                              a.Kin, MODE, BITS, F16);
     if constexpr (BITS == 4) {
