@@ -1004,7 +1004,10 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM>())) void ggemm_wr_k
           if constexpr (q == 0) sb_copy(kt0 / 4 + 1);
           __builtin_amdgcn_sched_barrier(0);
           compute(std::integral_constant<int, 1>{}, A, fb, rw[q], fsc[c], fbi[c], rw[(q + 1) % 4], fsc[n],
-                  fbi[n], An, kt + 1, [&] { bload(rw[(q + 2) % 4], kt + 2); });
+                  fbi[n], An, kt + 1, [&] {
+                    __builtin_amdgcn_sched_barrier(0);  // copies first: the wait below counts what follows them
+                    bload(rw[(q + 2) % 4], kt + 2);
+                  });
           // This wave's copies are done (only the 2 RL weight loads issued
           // after them may be outstanding), then every wave's.
           if constexpr (RL == 1)

@@ -307,8 +307,11 @@ __global__ __launch_bounds__(512) void router_topk16_kernel(const uint16_t* __re
   };
   auto slot = [&](int q, int s) { return (((4 * q + b) * SEG + s + i16) & 31) * 8; };
   // Ring order: tokens, then expert tiles 0 .. NT-1. Rows are private to the
-  // wave, so its own wait for its copies is enough.
+  // wave, so its own wait for its copies is enough. The counted wait takes the
+  // token rows to be the older eight, so nothing may move across the line
+  // between the two.
   copy16(rx, s_r0[wave], 0);
+  __builtin_amdgcn_sched_barrier(0);
   copy16(rw, s_r1[wave], 0);
   asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
   uint4 xr[2][SEG];
