@@ -682,6 +682,11 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM>())) void ggemm_wr_k
   // raw weights: the next one's are requested halfway through sub-step 1, when
   // half of this one's are used up, and A fragments are read two pairs ahead.
   constexpr bool LATE = BM == 128 && NJ == 4;
+  // A fragments read ahead of the MFMAs that use them, in row blocks. Two where
+  // a third does not fit: 8-bit half down and plain tiles of 64 rows spilled 2 to
+  // 12 of their 128 registers with three, and a reload from scratch memory waits
+  // for every load in flight.
+  constexpr int AHEAD = LATE || (BM == 64 && BITS == 8 && F16 && MODE != kGgGateUp) ? 2 : 3;
   using op_t = op8_t<F16>;
   using f16tag = std::integral_constant<bool, F16>;
   using D8 = Deq8<BITS, F16>;
@@ -902,7 +907,7 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM>())) void ggemm_wr_k
                      const sb_t* bic, uint4 (*rn)[RL], const sb_t* sn, const sb_t* bin, uint16_t* An,
                      int ktn, auto weight_load) __attribute__((always_inline)) {
     constexpr int MBL = decltype(mbl_tag)::value;
-    constexpr int NQ = 4 * MBL, D = LATE ? 2 : 3, R = D + 1;
+    constexpr int NQ = 4 * MBL, D = AHEAD, R = D + 1;
     constexpr int CR = 4 * WAVES;  // rows per copy round
     constexpr int NC = (16 * MBL + CR - 1) / CR < LA ? (16 * MBL + CR - 1) / CR : LA;
     constexpr int STEP = NQ / (2 * NC) > 0 ? NQ / (2 * NC) : 1;
