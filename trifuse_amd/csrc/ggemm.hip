@@ -1187,7 +1187,8 @@ struct WrTile {
 //  * Gate/up and gathered products. 64 rows up to a = 44 wide, 56 otherwise
 //    (OLMoE 300 tokens 49.0 against 54.6 on 128x8, 400 tokens 66.0 and 56.7;
 //    Granite 256 tokens, a = 51, 21.8 and 23.7; 8-bit codes 400 tokens 63.0
-//    and 73.6, so to a = 56 there), with 8 waves while that gives two tiles a
+//    and 73.6, so to a = 56 there, but to 48 with half storage, whose affine
+//    routers spread the loads more: 400 tokens 84.6 and 75.2), with 8 waves while that gives two tiles a
 //    compute unit and most experts have a route, else 4 (8-bit codes at 8
 //    tokens 39.5 against 47.4, at 20 tokens 53.8 and 53.5).
 //    128 rows to a = 232 wide (1700 tokens, a = 212: 138.8 against 153.3 on
@@ -1228,7 +1229,7 @@ static WrTile wr_tile(int64_t n_routes, int E, int64_t cols, int kin, int mode, 
       if (n_routes >= (int64_t)E * 448 && kin >= 1024) return {256, 8, 2};
       return {128, 4, 2};
     }
-    if (upto(wide && bits == 4 ? 44 : 56))
+    if (upto(!wide ? 56 : bits == 4 ? 44 : f16 ? 48 : 56))
       return {64, n_routes > 2 * E && E * mtiles(64) * cols >= 2 * cus ? 8 : 4, 2};
     if (mode == kGgGateUp && bits == 4 && !f16) {
       if (wide && (upto(96) || (!upto(112) && upto(400)))) return {128, 4, 4};
@@ -1239,9 +1240,20 @@ static WrTile wr_tile(int64_t n_routes, int E, int64_t cols, int kin, int mode, 
     }
     // 256-row tiles in one round of the compute units where 128-row ones need
     // more (Granite 700 tokens, a = 140: 35.1 against 38.8 on 128x4; 8-bit codes
-    // 1000 tokens 45.5 and 49.6).
-    if (!wide && E * mtiles(128) * cols > cus && E * mtiles(256) * cols <= cus) return {256, 8, 2};
+    // 1000 tokens 45.5 and 49.6). With long and short tiles the live rows may
+    // take at most 5/8 of their places: an XCD's run holds a tile or two more than an even share, and where
+    // no tile is short that is a second round (64 experts 512 -> 2 x 256, a = 375: half
+    // 34.1, bf16 45.8 for 8-bit codes, against 29.4 and 31.7 on 128x8; a = 275, whose
+    // second tiles are nearly empty: 25.9 and 29.3 on 128x4).
+    const int64_t live = (n_routes + (int64_t)E * 64 - 1) / ((int64_t)E * 64) * 64 * E * cols;
+    if (!wide && E * mtiles(128) * cols > cus && E * mtiles(256) * cols <= cus &&
+        (mtiles(256) == 1 || 8 * live <= 5 * 256 * cus))
+      return {256, 8, 2};
     if (n_routes >= (int64_t)E * (wide ? 232 : 480)) return {256, 8, 2};
+    // Eight waves also where their 128-row tiles take one well-filled round
+    // (Granite 600 tokens: half 29.4 on 128x4 and 27.0, 8-bit codes 34.9 and 33.0).
+    const int64_t round = E * mtiles(128) * cols;
+    if (mode == kGgGateUp && !wide && 8 * round >= 5 * cus && round <= cus) return {128, 8, 2};
     return {128, upto(104) ? 8 : 4, 2};
   };
   const WrTile t = pick();
@@ -1312,6 +1324,41 @@ static void launch_wr(const GgArgs& a, int64_t n_routes, int E, hipStream_t s) {
   tfm_launch(ggemm_wr_kernel<BM, MODE, BITS, F16, WV, false, NJ>, grid, WV * 64, 0, s, a);
 }
 
+// 8-bit codes with bf16 storage, inputs up to 2048 wide: where the 256-row tiles
+// of ggemm_kernel beat ggemm_wr_kernel. A code costs two to three vector
+// instructions there either way, but a wave of 128 x 64 outputs reads a
+// third less LDS than eight waves that each read the whole activation tile. us,
+// ggemm_kernel against the tile wr_tile picks, a = routes per expert:
+//  * Down and gathered products from a = 384, with more than half a round of the
+//    compute units in full tiles: OLMoE 3072 tokens 139 and 154, 3600 158
+//    and 174, Granite 2200 47 and 55, 6000 114 and 125; 16 experts 384 ->
+//    768 at 4096 tokens 21 and 28. Fewer tiles leave too much idle
+//    (16 experts 2048 -> 1024, 3072 tokens: 50 and 38; 2048 x 2048 linear, 4096
+//    rows: 54 and 43). Not around a = 512, where
+//    many experts start a third tile (Granite 2500 tokens 64 and 59).
+//  * Gathered products from a = 57 to 150 with two rounds of 128-row tiles: 64
+//    experts 1408 -> 2048, 4000 rows 70.1 and 72.6, 8000 rows 103.7 and 112.0;
+//    12000 rows level, and 2048 -> 1408 133.7 and 126.4.
+//  * Gate/up from 384 to 480 where two tiles an expert fill their rounds: OLMoE
+//    3600 tokens 260 and 270, 32 experts 1024 -> 2 x 512 at 3500 tokens 39 and
+//    49; Granite (320 tiles in two rounds) level. Beyond, level or up to 4%
+//    slower (OLMoE 6000 tokens 421 and 406), except with few column tiles (16
+//    experts 768 -> 2 x 384 at 4096 tokens 30 and 39).
+static bool lds_dequant(int64_t n_routes, int E, int64_t cols, int kin, int mode) {
+  if (kin > kLdsScaleKin || tile_override() || waves_override() || (mode == kGgDown && down_tile_override())) return false;
+  const int64_t cus = gg_device_cus();
+  auto avg = [&](int a) { return n_routes >= (int64_t)E * a; };
+  const bool tall = avg(384) && 2 * n_routes * cols > 256 * cus;
+  if (mode == kGgGateUp) {
+    const int64_t tiles = 2 * E * cols;
+    return tall && (4 * E * cols < cus || (!avg(480) && 4 * tiles >= 3 * ((tiles + cus - 1) / cus) * cus));
+  }
+  if (mode == kGgPlain && avg(57) && !avg(150) &&
+      (n_routes + (int64_t)E * 128 - 1) / ((int64_t)E * 128) * E * cols >= 2 * cus)
+    return true;
+  return tall && !(avg(480) && !avg(528));
+}
+
 // Inputs a multiple of 128 wide: weights in registers (ggemm_wr_kernel);
 // otherwise (odd multiples of 64, or scales or biases off a 4-byte boundary,
 // which only 2-byte loads reach) ggemm_kernel.
@@ -1320,9 +1367,10 @@ static void launch_tile(const GgArgs& a_in, int64_t n_routes, int E, hipStream_t
   GgArgs a = a_in;
   const uintptr_t sb = sb_address_bits(a);
   a.sb16 = (sb & 15) == 0 && a.Kin / BK % 8 == 0;
-  if (a.Kin % BK2 == 0 && (sb & 3) == 0) {
-    const WrTile t = wr_tile(n_routes, E, MODE == kGgGateUp ? (2 * (int64_t)a.N + 255) / 256 : ((int64_t)a.N + 255) / 256,
-                             a.Kin, MODE, BITS, F16);
+  const int64_t cols = ((MODE == kGgGateUp ? 2 : 1) * (int64_t)a.N + 255) / 256;
+  const bool lds = BITS == 8 && !F16 && (sb & 15) == 0 && lds_dequant(n_routes, E, cols, a.Kin, MODE);
+  if (a.Kin % BK2 == 0 && (sb & 3) == 0 && !lds) {
+    const WrTile t = wr_tile(n_routes, E, cols, a.Kin, MODE, BITS, F16);
     if constexpr (BITS == 4) {
       if (t.bm == 96) {
         launch_wr<96, MODE, BITS, F16, 4, 4>(a, n_routes, E, s);
