@@ -251,6 +251,28 @@ static bool ds_prefetch() {
   return v;
 }
 
+// Tokens up to which the grouped path runs the router as a logits kernel and a
+// top-k kernel (one wave a (token, expert) pair spreads the router over the
+// chip: logits, top-k and scatter 14.3 us at 45 tokens, against 16.3 for the
+// fused router kernel and its scatter, and 5 us less a layer; at 100 tokens level,
+// at 512 22.6 and 17.2). Unset 64, and whatever the tokens at up to 256 routes,
+// where top-k and grouping are one kernel; TFM_ROUTER_SPLIT_MAX_TOKENS sets the
+// tokens alone.
+static bool router_split(int T, int64_t R) {
+  static const int v = [] {
+    const char* s = std::getenv("TFM_ROUTER_SPLIT_MAX_TOKENS");
+    if (!s) return -1;
+    char* end = nullptr;
+    const long n = std::strtol(s, &end, 10);
+    if (!end || end == s || *end != 0 || n < 0 || n > (1 << 30)) {
+      std::fprintf(stderr, "trifuse_moe: ignoring invalid TFM_ROUTER_SPLIT_MAX_TOKENS=%s\n", s);
+      return -1;
+    }
+    return (int)n;
+  }();
+  return v >= 0 ? T <= v : T <= 64 || R <= 256;
+}
+
 static bool fused_decode(const tfm_geometry& g, int64_t R) {
   return R <= 256 && g.hidden_size <= 2048 && g.intermediate_size <= 2048;
 }
@@ -898,11 +920,7 @@ static void moe_forward_body(const tfm_plan* plan, const void* x, int64_t tokens
       launch_dequant_router(f16, weights->router_bits, weights->router_affine, E, H, ws.router_w, s);
       rw = ws.router_w;
     }
-    // Past 64 tokens; up to there one wave a (token, expert) pair spreads the
-    // router over the chip (logits, top-k and scatter 14.3 us at 45 tokens,
-    // against 16.3 for this kernel and its scatter, and 5 us less a layer; at
-    // 100 tokens level, at 512 22.6 and 17.2).
-    if (T > 64 && R > 256)
+    if (!router_split(T, R))
       fused_route = launch_router_topk(g.route, f16, static_cast<const uint16_t*>(x), rw, weights->logit_bias,
                                        T, H, E, K, ws.idx, ws.gates, ws.hist, s);
     if (!fused_route)

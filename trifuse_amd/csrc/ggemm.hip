@@ -39,6 +39,7 @@
 // in a private LDS block, 32 rows at a time, and writes them out as 16-byte
 // row chunks: h rows (gate/up), expert-output rows in sorted order (down) or
 // rows scattered to their flat route (gather_qmm).
+#include <cstdio>
 #include <cstdlib>
 #include <type_traits>
 
@@ -1109,20 +1110,19 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM>())) void ggemm_wr_k
   });
 }
 
+static int tile_rows_env(const char* name) {
+  const char* s = std::getenv(name);
+  const int n = s ? std::atoi(s) : 0;
+  return n == 64 || n == 96 || n == 128 || n == 256 ? n : 0;
+}
+
 static int tile_override() {
-  static int v = [] {
-    const char* s = std::getenv("TFM_GGEMM_TILE");
-    return s ? std::atoi(s) : 0;
-  }();
+  static const int v = tile_rows_env("TFM_GGEMM_TILE");
   return v;
 }
 
 static int down_tile_override() {
-  static int v = [] {
-    const char* s = std::getenv("TFM_GGEMM_DOWN_TILE");
-    const int n = s ? std::atoi(s) : 0;
-    return n == 64 || n == 96 || n == 128 || n == 256 ? n : 0;
-  }();
+  static const int v = tile_rows_env("TFM_GGEMM_DOWN_TILE");
   return v;
 }
 
@@ -1211,7 +1211,7 @@ struct WrTile {
 //    has too few registers for it.)
 // TFM_GGEMM_TILE=64/96/128/256 forces the rows, TFM_GGEMM_DOWN_TILE those of the
 // down GEMM alone (TFM_GGEMM_TILE takes precedence), TFM_GGEMM_WAVES=4/8 the
-// waves.
+// waves (of tiles of 64 or 128 rows that do not have that many already).
 static WrTile wr_tile(int64_t n_routes, int E, int64_t cols, int kin, int mode, int bits, bool f16) {
   const int64_t cus = gg_device_cus();
   auto mtiles = [&](int bm) { return (n_routes + (int64_t)E * bm - 1) / ((int64_t)E * bm); };
@@ -1258,9 +1258,9 @@ static WrTile wr_tile(int64_t n_routes, int E, int64_t cols, int kin, int mode, 
   };
   const WrTile t = pick();
   int bm = tile_override();
-  if (bm != 64 && bm != 96 && bm != 128 && bm != 256) bm = mode == kGgDown ? down_tile_override() : 0;
+  if (!bm) bm = mode == kGgDown ? down_tile_override() : 0;
   const int wv = waves_override();
-  if (!bm && !wv) return t;
+  if ((!bm || bm == t.bm) && (!wv || wv == t.wv)) return t;
   if (!bm) bm = t.bm;
   if (bm == 96) return {96, 4, 4};
   if (bm == 256) return {256, 8, 2};
@@ -1427,7 +1427,19 @@ static void launch_mode(const GgArgs& a, int bits, bool f16, int64_t n_routes, i
     ggemm_run_4_0(MODE, a, n_routes, E, s);
 }
 
+// TFM_GGEMM_SB_LAYOUT chose between layouts of whole-width scales in LDS. The
+// four-super-step ring has one, so the variable is accepted and said to do nothing.
+static void note_sb_layout() {
+  static const bool noted = [] {
+    const char* s = std::getenv("TFM_GGEMM_SB_LAYOUT");
+    if (s) std::fprintf(stderr, "trifuse_moe: TFM_GGEMM_SB_LAYOUT=%s has no effect (scales and biases have one layout)\n", s);
+    return s != nullptr;
+  }();
+  (void)noted;
+}
+
 static void check_shapes(int N, int Kin, int bits, int64_t x_rows) {
+  note_sb_layout();
   if (bits != 4 && bits != 8) fail(TFM_E_UNSUPPORTED, "grouped GEMM: weights must be 4-bit or 8-bit");
   if (Kin % BK != 0) fail(TFM_E_UNSUPPORTED, "grouped GEMM: input width must be a multiple of 64");
   if (N % 64 != 0) fail(TFM_E_UNSUPPORTED, "grouped GEMM: output width must be a multiple of 64");
