@@ -989,7 +989,7 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM>())) void ggemm_wr_k
   };
   if (FEW && rows_valid <= 16 && (KT & 3) == 0) {
     if constexpr (FEW) {
-      static_assert(BM == 64, "few-row tiles are 64-row tiles");
+      static_assert(BM == 64 && RL == 1 && NJ == 2, "few-row tiles: 64 rows, two weight loads a super-step");
       uint4 rw[4][NJ][RL];                         // raw weights of super-step k in slot k % 4
       sb_t fsc[2][NJ], fbi[2][NJ];                  // scales and biases of super-step k in set k % 2
       op_t fb[NJ];
@@ -1014,12 +1014,9 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM>())) void ggemm_wr_k
                     __builtin_amdgcn_sched_barrier(0);  // copies first: the wait below counts what follows them
                     bload(rw[(q + 2) % 4], kt + 2);
                   });
-          // This wave's copies are done (only the 2 RL weight loads issued
-          // after them may be outstanding), then every wave's.
-          if constexpr (RL == 1)
-            asm volatile("s_waitcnt vmcnt(2)\n\ts_barrier" ::: "memory");
-          else
-            asm volatile("s_waitcnt vmcnt(4)\n\ts_barrier" ::: "memory");
+          // This wave's copies are done (only the NJ weight loads issued after
+          // them may be outstanding), then every wave's.
+          asm volatile("s_waitcnt vmcnt(2)\n\ts_barrier" ::: "memory");
         });
       }
     }

@@ -321,18 +321,17 @@ void launch_group_scatter(const int32_t* ids, int64_t n, int E, int chunk, int32
     launch_group_empty(E, g, status, s);
     return;
   }
-  const int nsb = (nb + kSuperChunks - 1) / kSuperChunks;
   // Superblock sums live after the chunk histograms (group_hist_rows rows).
   // Up to kScatterChunks chunks the scatter kernel sums the histograms itself
   // (bsum null), which saves a dependent launch.
   int32_t* bsum = nullptr;
   if (nb > kScatterChunks) {
     bsum = hist + (int64_t)(nb + 1) * (E + 1);
-    superblock_sums_kernel<<<nsb, 64, 0, s>>>(hist, nb, E, bsum);
+    superblock_sums_kernel<<<(nb + kSuperChunks - 1) / kSuperChunks, 64, 0, s>>>(hist, nb, E, bsum);
     check_hip(hipGetLastError(), "group superblock sums launch");
   }
-  // One wave per workgroup where the chunk and the rows to sum are few.
-  if (chunk <= 64 && (bsum ? nsb : nb) <= 16)
+  // One wave per workgroup where the chunk and the histograms to sum are few.
+  if (chunk <= 64 && nb <= 16)
     tfm_launch(scatter_kernel<64>, nb, 64, 0, s, ids, n, E, chunk, hist, bsum, nb, g, status);
   else
     tfm_launch(scatter_kernel<kScatterThreads>, nb, kScatterThreads, 0, s, ids, n, E, chunk, hist, bsum, nb, g, status);
