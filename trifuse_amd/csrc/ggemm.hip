@@ -1198,7 +1198,7 @@ struct WrTile {
 //    71.8 and 78.3).
 //  * Gate/up of 4-bit codes with bf16 storage: 128 x 4 with 64 weight rows a
 //    wave, against the tile above: wide 700 tokens (a = 87) 66.9 and 71.6, 800
-//    tokens 78.0 and 75.8, 1000 tokens 104.0 and 106.5, 1300 tokens 120.6 and
+//    tokens 69.6 and 77.0, 860 tokens 84.5 and 87.7, 1000 tokens 104.0 and 106.5, 1300 tokens 120.6 and
 //    131.6, 1750 tokens 130.2 and 144.0, 2400 tokens 178.3 and 187.7, 4000
 //    tokens 277.0 and 271.6 (256x8). Not wide, where its rounds are full
 //    enough: Granite 1024 tokens (a = 205, 336 tiles in a round of 512) 47.8
@@ -1229,7 +1229,7 @@ static WrTile wr_tile(int64_t n_routes, int E, int64_t cols, int kin, int mode, 
     if (upto(!wide ? 56 : bits == 4 ? 44 : f16 ? 48 : 56))
       return {64, n_routes > 2 * E && E * mtiles(64) * cols >= 2 * cus ? 8 : 4, 2};
     if (mode == kGgGateUp && bits == 4 && !f16) {
-      if (wide && (upto(96) || (!upto(112) && upto(400)))) return {128, 4, 4};
+      if (wide && upto(400)) return {128, 4, 4};
       // Tiles of E experts of a / 128 + 1/2 m-tiles, two a compute unit: the
       // rounds must be two thirds full.
       const int64_t tiles = (n_routes + (int64_t)E * 64) * cols / 128, round = 2 * cus;
