@@ -540,25 +540,25 @@ __global__ __launch_bounds__(WAVES_M_ * WAVES_N_ * 64, 1) void ggemm_kernel(GgAr
 // 4- and 8-bit weights with inputs a multiple of 128 wide: the weights stay
 // in registers.
 //
-// Tile: BM routed rows x 256 weight rows, eight waves. Wave w owns 32 weight
-// rows (gate/up: gate rows 16w..16w+15 and the same up rows; down and plain:
-// rows 32w..32w+31) for all BM rows, as 16 x 16 blocks of
-// v_mfma_f32_16x16x32_bf16 (or _f16): BM/16 row blocks x 2 column blocks,
-// 4 fp32 accumulators each per lane. A gate block and its up block sit in
-// the same lanes, so SwiGLU needs no exchange.
+// Tile: BM routed rows x 16 NJ WV weight rows, WV (4 or 8) waves. Wave w owns
+// 16 NJ (32 or 64) weight rows for all BM rows (gate/up: gate rows 8 NJ w ..
+// + 8 NJ - 1 and the same up rows; down and plain: rows 16 NJ w .. + 16 NJ - 1),
+// as 16 x 16 blocks of v_mfma_f32_16x16x32_bf16 (or _f16): BM/16 row blocks x
+// NJ column blocks, 4 fp32 accumulators each per lane. A gate block and its
+// up block sit in the same lanes, so SwiGLU needs no exchange.
 //
 // Per super-step of 128 k (two quantisation groups):
 //   * the BM activation rows are copied into LDS (one of two stages);
 //   * lane l loads the 32 contiguous codes (16 or 32 bytes) k = 32 (l / 16)
-//     .. + 31 of the super-step of each of its two weight rows; they share one
+//     .. + 31 of the super-step of each of its NJ weight rows; they share one
 //     scale group. Codes 8 s .. 8 s + 7 of them are dequantised into the B
 //     operand of sub-step s. The reduction order inside an MFMA is free, so
 //     the A operand of sub-step s for lane l is the same k range: LDS chunk
 //     4 (l / 16) + s of the row;
 //   * one barrier, for the next stage's activations.
 // Every packed weight is dequantised exactly once per tile and never goes
-// through LDS. Per 128 k a wave runs 4 x BM/8 MFMAs for one barrier, twice the
-// work per barrier of the kernel above.
+// through LDS. Per 128 k a wave runs 4 NJ x BM/16 MFMAs for one barrier: twice
+// the work per barrier of the kernel above at the same tile.
 //
 // LDS: activation row r of a stage is 256 B (16 chunks of 16 B); chunk c is
 // stored in slot c ^ (r & 15), so the 16 lanes of one read pass (16
@@ -893,8 +893,8 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM>())) void ggemm_wr_k
   // super-step's raw weights). The (sub-step, row block) pairs run as one
   // compile-time sequence with the A fragment of pair q + D read while pair
   // q computes (a ring of D + 1 fragments); the scheduler is asked for the
-  // first D reads, then per pair two MFMAs, the read D pairs ahead and three
-  // VALU instructions. The activation copies of the next super-step (into
+  // first D reads, then per pair the read D pairs ahead, NJ MFMAs and its share
+  // of the dequantisation slices. The activation copies of the next super-step (into
   // stage An) are issued one every STEP pairs over the first half of the
   // sequence: issued together they would hold the wave at the address unit,
   // with no MFMAs issued, for most of a thousand cycles. Only the NC copies
@@ -951,17 +951,6 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM>())) void ggemm_wr_k
     });
   };
 
-  // ---- few rows (FEW instances): weights two super-steps ahead ----
-  // In the loop below every super-step ends at a barrier that waits for all
-  // of its loads, and the raw weights of super-step k+1 (whose first word
-  // the last sub-step of super-step k dequantises) are requested at the start
-  // of super-step k: one super-step of loads in flight. A tile of at most 16
-  // rows (one row block) has too few MFMAs per super-step to cover a memory
-  // latency that way. Here the raw weights of super-step k+2 are requested
-  // right after the activation copy of super-step k+1, and the barrier waits
-  // only for that copy (the vector memory counter retires in issue order), so
-  // they stay in flight across it. The products and their order are those of
-  // the loop below.
   // Live row blocks (uniform over the workgroup), so that empty rows cost no
   // MFMAs: in steps of four of 16 blocks, of two of 8; 2, 4, 5 or 6 with 96-row
   // tiles; 1, 2 or 4 with 64-row ones (16, 32 or 64 rows).
@@ -987,6 +976,17 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM>())) void ggemm_wr_k
       else f(std::integral_constant<int, 1>{});
     }
   };
+  // ---- few rows (FEW instances): weights two super-steps ahead ----
+  // In the main loop every super-step ends at a barrier that waits for all
+  // of its loads, and the raw weights of super-step k+1 (whose first word
+  // the last sub-step of super-step k dequantises) are requested at the start
+  // of super-step k: one super-step of loads in flight. A tile of at most 16
+  // rows (one row block) has too few MFMAs per super-step to cover a memory
+  // latency that way. Here the raw weights of super-step k+2 are requested
+  // right after the activation copy of super-step k+1, and the barrier waits
+  // only for that copy (the vector memory counter retires in issue order), so
+  // they stay in flight across it. The products and their order are those of
+  // the main loop.
   if (FEW && rows_valid <= 16 && (KT & 3) == 0) {
     if constexpr (FEW) {
       static_assert(BM == 64 && RL == 1 && NJ == 2, "few-row tiles: 64 rows, two weight loads a super-step");
@@ -1059,9 +1059,9 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM>())) void ggemm_wr_k
   // ---- epilogue ----
   // Rows staged row-major, CP columns per pass (the first BM/2 rows in
   // stage 0, the rest in stage 1), then written as 16-byte row pieces.
-  // Gate/up: one pass of BN/2 columns (wave w holds columns 16w..16w+15
-  // after SwiGLU); down and plain: BN/128 passes of 128 columns, waves
-  // 4p..4p+3 staging columns 128p..128p+127.
+  // Gate/up: one pass of BN/2 columns (wave w holds columns 8 NJ w .. + 8 NJ - 1
+  // after SwiGLU); down and plain: BN/128 passes of 128 columns, pass p staged
+  // by the waves that hold columns 128p..128p+127 (four of 32, two of 64).
   constexpr int PASSES = MODE == kGgGateUp ? 1 : BN / 128;
   constexpr int CP = MODE == kGgGateUp ? BN / 2 : 128;
   constexpr int PARTS = CP / 8;                   // 16-byte pieces per staged row
@@ -1185,9 +1185,10 @@ struct WrTile {
 //    (OLMoE 300 tokens 49.0 against 54.6 on 128x8, 400 tokens 66.0 and 56.7;
 //    Granite 256 tokens, a = 51, 21.8 and 23.7; 8-bit codes 400 tokens 63.0
 //    and 73.6, so to a = 56 there, but to 48 with half storage, whose affine
-//    routers spread the loads more: 400 tokens 84.6 and 75.2), with 8 waves while that gives two tiles a
-//    compute unit and most experts have a route, else 4 (8-bit codes at 8
-//    tokens 39.5 against 47.4, at 20 tokens 53.8 and 53.5).
+//    routers spread the loads more: 400 tokens 84.6 and 75.2), with 8 waves
+//    while that gives two tiles a compute unit and most experts have a route,
+//    else 4 (8-bit codes at 8 tokens 39.5 against 47.4, at 20 tokens 53.8 and
+//    53.5).
 //    128 rows to a = 232 wide (1700 tokens, a = 212: 138.8 against 153.3 on
 //    256x8; 2048 tokens, a = 256: 170.9 and 160.5), 480 otherwise (Granite
 //    1500 tokens, a = 300: 54.0 and 62.0; 2800, a = 560: 93.7 and 84.9): the
@@ -1198,14 +1199,17 @@ struct WrTile {
 //    71.8 and 78.3).
 //  * Gate/up of 4-bit codes with bf16 storage: 128 x 4 with 64 weight rows a
 //    wave, against the tile above: wide 700 tokens (a = 87) 66.9 and 71.6, 800
-//    tokens 69.6 and 77.0, 860 tokens 84.5 and 87.7, 1000 tokens 104.0 and 106.5, 1300 tokens 120.6 and
-//    131.6, 1750 tokens 130.2 and 144.0, 2400 tokens 178.3 and 187.7, 4000
+//    tokens 69.6 and 77.0, 860 tokens 84.5 and 87.7, 1000 tokens 104.0 and 106.5,
+//    1300 tokens 120.6 and 131.6, 1750 tokens 130.2 and 144.0, 2400 tokens 178.3 and 187.7, 4000
 //    tokens 277.0 and 271.6 (256x8). Not wide, where its rounds are full
 //    enough: Granite 1024 tokens (a = 205, 336 tiles in a round of 512) 47.8
 //    and 43.4, 1500 tokens (454) 51.2 and 54.5, 2048 tokens (592 in two) 10 us
 //    a layer slower, 2500 tokens (704) 74.6 and 84.5, 4000 tokens (1080 in
 //    three) 114.9 and 123.9. (The down GEMM is level or slower on it; half storage
 //    has too few registers for it.)
+// The lines were drawn at those two sizes. 840 calls at ten more (8 to 64
+// experts, 256 to 8192 wide) take 0.79 of the time they took under the rule
+// before it (geometric mean), the slowest 1.09.
 // TFM_GGEMM_TILE=64/96/128/256 forces the rows, TFM_GGEMM_DOWN_TILE those of the
 // down GEMM alone (TFM_GGEMM_TILE takes precedence), TFM_GGEMM_WAVES=4/8 the
 // waves (of tiles of 64 or 128 rows that do not have that many already).

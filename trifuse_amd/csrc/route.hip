@@ -120,9 +120,10 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const uint16_t* __re
 //
 // Bound: 2 E H flop per token at 256 flop per clock and compute unit in the
 // 16 x 16 form (the 4 x 4 form measured about a quarter of that), and the E H
-// x 2 bytes of router rows per workgroup from L2. Up to 1024 tokens the 4-token
-// form fills the chip and the few products are not its bound; beyond, 16
-// tokens read the router a quarter as often.
+// x 2 bytes of router rows per workgroup from L2. The 4-token form runs up to
+// 1024 tokens, in one round of one workgroup a compute unit (75 workgroups at
+// 300 tokens, 256 at 1024), where latency and not the few products is the bound;
+// beyond, 16 tokens read the router a quarter as often.
 __device__ __forceinline__ void route_dma16(__amdgpu_buffer_rsrc_t r, uint16_t* dst, uint32_t voff) {
 #if defined(__HIP_DEVICE_COMPILE__)
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, voff, 0, 0, 0);
