@@ -713,7 +713,7 @@ __global__ __launch_bounds__(256) void olmoe_softmax_kernel(const uint16_t* __re
   const float ld = valid ? st2f<F16>(logits[(int64_t)t * E + lane]) : -__builtin_inff();
   float norm;
   const float ex = wave_softmax_exp(ld, &norm);
-  if (valid) probs[(int64_t)t * E + lane] = f2st<F16>(ex * norm);
+  if (valid) probs[(int64_t)t * E + lane] = f2st<F16>(softmax_prob(ex, norm));
 }
 
 void launch_olmoe_softmax(bool f16, const uint16_t* logits, int T, int E, uint16_t* probs, hipStream_t s) {
