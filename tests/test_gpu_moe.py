@@ -114,11 +114,12 @@ def test_granite_batch_sweep(gpu, T):
 
 
 @pytest.mark.parametrize("name", ["granite_t768", "olmoe_t1792"])
-def test_tall_tiles_below_384_routes(gpu, name):
-    """256-row grouped-GEMM tiles where experts average fewer than 384 routes:
-    Granite 768 tokens (154 per expert; 256-row tiles fit one round of the
-    compute units) and OLMoE 1792 tokens (224 per expert), every token
-    checked."""
+def test_large_tiles_below_384_routes(gpu, name):
+    """Large tiles where experts average fewer than 384 routes: Granite 768
+    tokens (154 per expert: 256-row gate/up tiles in one round of the compute
+    units, 128-row down tiles) and OLMoE 1792 tokens (224 per expert: 128-row
+    tiles, of 64 weight rows a wave for gate/up), every token checked.
+    256-row tiles past 232 routes per expert are in test_gpu_tiles.py."""
     w = wl.get_workload(name)
     log(f"moe {w.name}")
     layer = wl.workload_layers(w, gpu)[0]

@@ -5,18 +5,20 @@ import pytest
 import torch
 
 import oracle
-from tests._util import BLOCK_TOL, log, max_rel, u16, u32
+from tests._util import log, max_rel, u16, u32
 from trifuse_amd import moe as tmoe
 from trifuse_amd import workload as wl
 
 pytestmark = pytest.mark.gpu
 
 DT = {"bf16": torch.bfloat16, "f16": torch.float16}
-# A product's largest error over its largest value. A weight and the result
-# are each rounded to the storage type (half a step: 2^-9 of a bf16 value, 2^-12
-# of a half one). Weight errors add up as a random walk and stay below half a
-# step of the largest result; the fp32 sums add 1e-6. Twice the half step.
-STEP = {"bf16": 2.0 ** -8, "f16": 2.0 ** -11}
+# A product's largest error over its largest value, in half steps u of the storage
+# type (2^-8 of a bf16 value, 2^-11 of a half one). The result is rounded once:
+# at most u of the largest. Its weights are rounded to about 0.4 u each (rms), which
+# over a product adds up to 0.4 u of the result's rms, five times that at most over
+# some 10^6 results, whose largest is about five times their rms: 0.4 u of the
+# largest. The fp32 sums add 1e-6. So 1.4 u and a little.
+STEP = {"bf16": 1.5 * 2.0 ** -8, "f16": 1.5 * 2.0 ** -11}
 
 
 def _affine(shape, bits, dtype, key, device):
@@ -27,24 +29,53 @@ def _affine(shape, bits, dtype, key, device):
     return q, s, (s.float() * -float(2 ** (bits - 1))).to(DT[dtype])
 
 
+# Counts that end a 16-row block, a tile or its live-row steps exactly, one row
+# early and one row late.
+EDGES = [0, 1] + [c + d for c in (16, 32, 48, 64, 80, 96, 112, 128, 160, 192, 224, 256) for d in (-1, 0, 1)]
+
+
 def _routes(T, E, K, seed):
-    """K distinct experts a token: expert 0 for every other token (more rows
-    than one tile), expert 1 for none, the rest at random."""
-    rng = np.random.default_rng(seed)
-    score = rng.random((T, E))
-    score[::2, 0] = 2.0
-    score[:, 1] = -1.0
-    return np.argsort(-score, axis=1)[:, :K].astype(np.int32)
+    """T x K expert ids in random order: EDGES as the route counts of the first
+    experts, as far as they take two thirds of the routes, the rest shared out
+    evenly."""
+    counts, left = np.zeros(E, dtype=np.int64), T * K
+    for e, c in zip(range(E - 4), EDGES):
+        if 3 * (T * K - left + c) > 2 * T * K:
+            break
+        counts[e] = c
+        left -= c
+    rest = E - 1 - e
+    counts[e + 1:] = left // rest
+    counts[E - 1] += left - left // rest * rest
+    ids = np.repeat(np.arange(E, dtype=np.int32), counts)
+    np.random.default_rng(seed).shuffle(ids)
+    return ids.reshape(T, K)
 
 
-# Routes per expert on average, over the tile rule's lines: 64-, 96- and
-# 128-row tiles, two 96-row tiles, 128 and 256 rows.
+# Two and a half half steps of the storage type, as for products: the result is
+# rounded once (1), the K weighted expert outputs once each (less than 1), and the
+# rounded weights and hidden rows of three products average out (0.4 each, in
+# squares).
+BLOCK_STEPS = {"bf16": 1e-2, "f16": 1e-2 / 8}
+
+# Geometries with every input width an odd number of 128-wide super-steps or
+# output columns off the tile: experts x columns that fill the compute units (down
+# GEMM too), gate/up columns off the tile, and experts that do not fill them.
+WIDE, RAGGED, NARROW = (1152, 640, 64, 8), (640, 704, 64, 8), (384, 512, 40, 8)
+# Routes per expert on average, over the tile rule's lines: 64-, 96- and 128-row
+# tiles, two 96-row tiles, 128 and 256 rows; for few columns also both sides of
+# one round of 256-row tiles (128) and of the 64-weight-row tiles' fill (300).
+CASES = [(WIDE, a) for a in (6, 30, 47, 60, 90, 105, 140, 200, 260, 450)] + [(RAGGED, a) for a in (60, 90, 140)] + \
+    [(NARROW, a) for a in (10, 30, 58, 126, 130, 200, 300, 400, 500)]
+
+
 @pytest.mark.parametrize("dtype,bits", [("bf16", 4), ("f16", 4), ("bf16", 8), ("f16", 8)])
-@pytest.mark.parametrize("a", [6, 30, 60, 90, 105, 140, 200, 450])
-def test_block_tiles(gpu, dtype, bits, a):
-    H, I, E, K = 1024, 1024, 64, 8
+@pytest.mark.parametrize("geom,a", CASES, ids=[f"{g[0]}x{g[1]}-{a}" for g, a in CASES])
+def test_block_tiles(gpu, dtype, bits, geom, a):
+    """Every token of a block against the per-expert fp64 reference."""
+    H, I, E, K = geom
     T = a * E // K + 3
-    log(f"block tiles {dtype} bits={bits} a={a} T={T}")
+    log(f"block tiles {dtype} bits={bits} H={H} I={I} E={E} a={a} T={T}")
 
     class L:
         pass
@@ -62,11 +93,10 @@ def test_block_tiles(gpu, dtype, bits, a):
     wts = tmoe.ExpertWeights(None, *w["gate"], *w["up"], *w["down"])
     y = blk.experts(x.to(gpu), torch.from_numpy(idx).to(gpu), torch.from_numpy(gates).to(gpu), wts)
     torch.cuda.synchronize()
-    pick = np.unique(np.concatenate([np.arange(4), np.linspace(0, T - 1, 12).astype(np.int64), [T - 1]]))
-    ref = oracle.moe_reference(u16(x)[pick], idx[pick], gates[pick], lay, dtype=dtype)
-    err = max_rel(oracle.st_to_f32(u16(y)[pick], dtype), ref)
+    ref = oracle.moe_reference_full(u16(x), idx, gates, lay, dtype=dtype)
+    err = max_rel(oracle.st_to_f32(u16(y), dtype), ref)
     log(f"  max_rel {err:.2e}")
-    assert err <= BLOCK_TOL
+    assert err <= BLOCK_STEPS[dtype]
 
 
 # Input widths: odd multiples of 64 (the LDS-dequantising kernel), one
@@ -91,7 +121,7 @@ def test_product_shapes(gpu, dtype, bits, E, N, Kin, rows):
     ref = oracle.gather_qmm_f64(u16(x)[pick], np.arange(pick.size), rhs[pick], u32(q), u16(s), u16(b), dtype=dtype)
     err = max_rel(oracle.st_to_f32(u16(out)[pick], dtype), ref)
     log(f"  max_rel {err:.2e}")
-    assert err <= BLOCK_TOL
+    assert err <= STEP[dtype]
 
 
 def _shifted(t, elements):
@@ -157,6 +187,42 @@ def test_prefill_router(gpu, route, H, E, T):
         np.testing.assert_array_equal(idx.cpu().numpy(), ridx)
         want = oracle.bf16_to_f32(rg) if route == "olmoe" else rg
         np.testing.assert_array_equal(gates.float().cpu().numpy(), want)
+
+
+# The same kernels on half storage, whose router is affine and dequantised first:
+# 4- and 16-token workgroups, half subnormals, infinities and NaN.
+@pytest.mark.parametrize("T", [65, 1024, 1025, 1043])
+@pytest.mark.parametrize("route,H,E,router_bits", [("olmoe", 2048, 64, 4), ("granite", 1536, 40, 4), ("olmoe", 1024, 49, 8),
+                                                   ("granite", 512, 7, 8)])
+def test_prefill_router_half(gpu, route, H, E, router_bits, T):
+    log(f"prefill router half {route} H={H} E={E} T={T} router bits={router_bits}")
+    I, K = 64, min(6, E)
+    x = wl.normal_bf16((T, H), 1.0, T + H, dtype=torch.float16)
+    x[1, 5] = float("inf")
+    x[2, 7] = float("nan")
+    x[3] = 5e-8  # one step of the half subnormals
+    x[4] = 0.0
+    x[5] = 3e-6
+    rq, rs, rb = _affine((E, H), router_bits, "f16", E + T, gpu)
+    rs, rb = rs * 0.3, rb * 0.3
+    rs[0], rb[0] = 2e-7, -1.5e-6  # subnormal weights
+    lb = wl.zipf_bias(E, 3)
+    blk = tmoe.MoEBlock(H, I, E, K, route=route, dtype=torch.float16, router="affine")
+    mk = [_affine((E, r, c), 4, "f16", 900 + r, gpu) for r, c in ((I, H), (I, H), (H, I))]
+    for bias in (None, lb):
+        wts = tmoe.ExpertWeights(None, *mk[0], *mk[1], *mk[2], router_q=rq, router_s=rs, router_b=rb, router_bits=router_bits,
+                                 logit_bias=None if bias is None else bias.to(gpu))
+        _, idx, gates = blk.forward(x.to(gpu), wts, return_routes=True)
+        torch.cuda.synchronize()
+        logits = oracle.router_logits_affine(u16(x), u32(rq), u16(rs), u16(rb), None if bias is None else bias.numpy(),
+                                             dtype="f16")
+        if route == "olmoe":
+            ridx, rg = oracle.route_olmoe(logits, K, dtype="f16")
+            rg = oracle.f16_to_f32(rg)
+        else:
+            ridx, rg = oracle.route_granite(logits, K, dtype="f16")
+        np.testing.assert_array_equal(idx.cpu().numpy(), ridx)
+        np.testing.assert_array_equal(gates.float().cpu().numpy(), rg)
 
 
 # One workgroup up to 1024 routes, chunk histograms read whole up to 256
