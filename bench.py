@@ -320,6 +320,23 @@ def gemv_gateup_label(g, T: int, bits: int) -> str:
     return "gemv_kernel<gateup>" if slots else "decode_gateup_kernel"
 
 
+def ggemm_gateup_label(g, routes: int, bits: int, dtype: str) -> str:
+    """The grouped GEMM's gate/up kernel: inputs a multiple of 128 wide run the
+    weights-in-registers kernel, others the LDS-dequantising one, which 8-bit
+    bf16 codes also take from 384 routes per expert while two 256-row tiles an
+    expert fill their rounds of the 256 compute units (any TFM_GGEMM_ override of
+    the tile keeps them on the former, as in the library)."""
+    E, cols, cus = g.experts, (2 * g.intermediate + 255) // 256, 256
+    lds = g.hidden % 128 != 0
+    forced = any(os.environ.get(k, "0") != "0" for k in ("TFM_GGEMM_TILE", "TFM_GGEMM_WAVES"))
+    if bits == 8 and dtype == "bf16" and g.hidden <= 2048 and not forced:
+        tall = routes >= 384 * E and 2 * routes * cols > 256 * cus
+        tiles = 2 * E * cols
+        fits = routes < 480 * E and 4 * tiles >= 3 * -(-tiles // cus) * cus
+        lds = lds or (tall and (4 * E * cols < cus or fits))
+    return "ggemm_kernel<gateup>" if lds else "ggemm_wr_kernel<gateup>"
+
+
 def dominant_roofline(r: Runner, stages):
     """Roofline object for the gate/up kernel (the largest share of bytes and FLOPs)."""
     from trifuse_amd import workload as wl
@@ -348,10 +365,7 @@ def dominant_roofline(r: Runner, stages):
             H % 512 == 0 and 512 <= H <= 2048 and I % 512 == 0 and 512 <= I <= 2048)
     streaming = fits and (T <= 3 or r.wl.bits != 4)
     gemv = gemv and not (fits and T <= 3)
-    # 4-bit weights with inputs up to 2048 wide (a multiple of 128) run the
-    # weights-in-registers grouped GEMM, everything else the LDS-dequant one
-    wr = r.wl.bits == 4 and H <= 2048 and H % 128 == 0
-    gemm_label = "ggemm_wr_kernel<gateup>" if wr else "ggemm_kernel<gateup>"
+    gemm_label = ggemm_gateup_label(g, R, r.wl.bits, r.wl.dtype)
     if is_decode(r.wl):
         # Per launch: routed experts' gate+up Q/S/B, x rows in, h rows out.
         per_launch = sum(u * gu_bytes_expert + T * H * 2 + T * g.top_k * I * 2 for u in U) / len(U)
