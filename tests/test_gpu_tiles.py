@@ -103,13 +103,15 @@ def test_block_tiles(gpu, dtype, bits, geom, a):
 # super-step, group counts not a multiple of 8 (4-byte scale copies), past
 # 2048; output widths off the tile; rows around 16, 32, 64, 96 and 128; the
 # lines between which 8-bit bf16 codes take the LDS-dequantising kernel (57, 384
-# and not 480 to 528 rows an expert).
+# and not 480 to 528 rows an expert); few rows an expert at one, three and, past
+# the scales that a tile keeps, five chunks of scales.
 @pytest.mark.parametrize("dtype,bits", [("bf16", 4), ("f16", 4), ("bf16", 8), ("f16", 8)])
 @pytest.mark.parametrize("E,N,Kin,rows", [(1, 64, 64, 200), (1, 192, 128, 177), (2, 320, 192, 500), (3, 128, 384, 401),
                                           (2, 192, 640, 290), (1, 256, 2304, 180), (40, 64, 1536, 41 * 17),
                                           (64, 1024, 128, 64 * 60), (64, 1024, 256, 64 * 110), (64, 1088, 128, 64 * 140),
                                           (64, 1024, 128, 64 * 250), (64, 2048, 128, 64 * 57), (16, 1536, 256, 16 * 383),
-                                          (16, 1536, 256, 16 * 384), (16, 1536, 256, 16 * 500), (16, 1536, 256, 16 * 530)])
+                                          (16, 1536, 256, 16 * 384), (16, 1536, 256, 16 * 500), (16, 1536, 256, 16 * 530),
+                                          (64, 2048, 512, 64 * 5), (64, 2048, 1536, 64 * 7), (64, 2048, 2560, 64 * 5)])
 def test_product_shapes(gpu, dtype, bits, E, N, Kin, rows):
     log(f"product {dtype} bits={bits} E={E} N={N} Kin={Kin} rows={rows}")
     q, s, b = _affine((E, N, Kin), bits, dtype, 7 * N + Kin + bits, gpu)

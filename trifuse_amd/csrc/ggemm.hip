@@ -564,7 +564,7 @@ __global__ __launch_bounds__(WAVES_M_ * WAVES_N_ * 64, 1) void ggemm_kernel(GgAr
 // stored in slot c ^ (r & 15), so the 16 lanes of one read pass (16
 // consecutive rows, one chunk) hit distinct bank groups. The scales and
 // biases of the tile's rows are kept for four super-steps at a time (eight
-// groups, 16 bytes a row) in a ring of two.
+// groups, 16 bytes a row) in a ring of two (few-row tiles of eight waves: four).
 constexpr int BK2 = 128;
 
 __device__ __forceinline__ f32x4_t mfma16(bf16x8_t a, bf16x8_t b, f32x4_t c, std::false_type) {
@@ -656,7 +656,7 @@ struct Deq8 {
 // Tile of BM = 64, 96, 128 or 256 rows by BN = 16 NJ WV weight rows. Where the
 // LDS and registers allow it, two or more workgroups share a compute unit, and
 // one covers the other's load latency, barriers and epilogue: 64 x 8 waves two
-// (48 KB, 128 registers), 64 x 4 four (40 KB), 96 x 4 (NJ = 4) and 128 x 4 two
+// (48 KB, 64 with few rows, 128 registers), 64 x 4 four (40 KB), 96 x 4 (NJ = 4) and 128 x 4 two
 // (64 and 72 KB, 256 registers), 128 x 8 and 256 x 8 one. WV = 4 with NJ = 2
 // halves the weight rows of a tile (128: 64 gate and 64 up rows, or 128 down
 // rows) for twice the tiles, where 8-wave tiles would leave compute units idle
@@ -697,7 +697,13 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM>())) void ggemm_wr_k
 
   __shared__ __attribute__((aligned(16))) uint16_t sA0[BM * BK2];
   __shared__ __attribute__((aligned(16))) uint16_t sA1[BM * BK2];
-  __shared__ __attribute__((aligned(16))) uint16_t sSb[2 * 2 * SBH];  // [ring slot][scale, bias][row][8 groups]
+  // Scale and bias chunks kept: a ring of two, or with few rows and eight waves
+  // (whose registers hold a compute unit to two workgroups, so the LDS has room)
+  // four, the whole of a 2048-wide input, copied before the loop. In the few-row
+  // loop nothing covers the memory latency of a copy: OLMoE 44 tokens 75.2 us a
+  // layer with the ring of two, 72.1 with all four ahead.
+  constexpr int SLOTS = FEW && WV == 8 ? 4 : 2;
+  __shared__ __attribute__((aligned(16))) uint16_t sSb[SLOTS * 2 * SBH];  // [slot][scale, bias][row][8 groups]
   // Tile prefix, XCD bounds and expert index: in activation stage 1, first
   // written after the prologue's barrier.
   int* const s_tiles = reinterpret_cast<int*>(sA1);
@@ -823,7 +829,7 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM>())) void ggemm_wr_k
   };
 
   // Scales and biases: chunk c holds groups 8c..8c+7 (super-steps 4c..4c+3) of
-  // the tile's BN rows, 16 bytes a row, in ring slot c % 2. The first half of
+  // the tile's BN rows, 16 bytes a row, in ring slot c % SLOTS. The first half of
   // the waves copies scales, the second biases, 64 rows each: one 16-byte
   // LDS-DMA per wave and chunk. Rows that start on 4-byte boundaries only (G
   // not a multiple of 8, or arrays off a 16-byte boundary) take four 4-byte
@@ -845,7 +851,7 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM>())) void ggemm_wr_k
       const auto rsb = gg_rsrc(static_cast<const char*>(sbias ? sm.biases : sm.scales) + (size_t)e * args.N * srow,
                                (uint32_t)args.N * srow);
       const int sn0 = n0 + 64 * sw - (sup ? BN / 2 : 0);  // matrix row of the first
-      uint16_t* const dst = sSb + ((c & 1) * 2 + (sbias ? 1 : 0)) * SBH + 64 * 8 * sw;
+      uint16_t* const dst = sSb + ((c & (SLOTS - 1)) * 2 + (sbias ? 1 : 0)) * SBH + 64 * 8 * sw;
       const bool live = 8 * c < G;
       if (sb16) {
         const int n = sn0 + lane;
@@ -863,7 +869,7 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM>())) void ggemm_wr_k
   auto sb_read = [&](sb_t* sc, sb_t* bi, int kt) {
     int g = 2 * kt + (g4 >> 1);
     g = g < G ? g : G - 1;
-    const uint16_t* const p = sSb + ((g >> 3) & 1) * 2 * SBH + (g & 7);
+    const uint16_t* const p = sSb + ((g >> 3) & (SLOTS - 1)) * 2 * SBH + (g & 7);
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
       sc[j] = D8::sb(p[trow[j] * 8]);
@@ -987,13 +993,14 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM>())) void ggemm_wr_k
   // only for that copy (the vector memory counter retires in issue order), so
   // they stay in flight across it. The products and their order are those of
   // the main loop.
-  if (FEW && rows_valid <= 16 && (KT & 3) == 0) {
+  if (FEW && rows_valid <= 16 && (KT & 3) == 0 && (SLOTS == 2 || KT <= 4 * SLOTS)) {
     if constexpr (FEW) {
       static_assert(BM == 64 && RL == 1 && NJ == 2, "few-row tiles: 64 rows, two weight loads a super-step");
       uint4 rw[4][NJ][RL];                         // raw weights of super-step k in slot k % 4
       sb_t fsc[2][NJ], fbi[2][NJ];                  // scales and biases of super-step k in set k % 2
       op_t fb[NJ];
-      sb_copy(0);
+#pragma unroll
+      for (int c = 0; c < (SLOTS == 2 ? 1 : SLOTS); ++c) sb_copy(c);
       a_copy(sA0, 0);
       bload(rw[0], 0);
       bload(rw[1], 1);
@@ -1007,7 +1014,7 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM>())) void ggemm_wr_k
           uint16_t* const A = c == 0 ? sA0 : sA1;
           uint16_t* const An = c == 0 ? sA1 : sA0;
           sb_read(fsc[n], fbi[n], kt + 1);
-          if constexpr (q == 0) sb_copy(kt0 / 4 + 1);
+          if constexpr (q == 0 && SLOTS == 2) sb_copy(kt0 / 4 + 1);
           __builtin_amdgcn_sched_barrier(0);
           compute(std::integral_constant<int, 1>{}, A, fb, rw[q], fsc[c], fbi[c], rw[(q + 1) % 4], fsc[n],
                   fbi[n], An, kt + 1, [&] {
