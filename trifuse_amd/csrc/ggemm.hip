@@ -1193,9 +1193,10 @@ struct WrTile {
 //    Granite 256 tokens, a = 51, 21.8 and 23.7; 8-bit codes 400 tokens 63.0
 //    and 73.6, so to a = 56 there, but to 48 with half storage, whose affine
 //    routers spread the loads more: 400 tokens 84.6 and 75.2), with 8 waves
-//    while that gives two tiles a compute unit and most experts have a route,
-//    else 4 (8-bit codes at 8 tokens 39.5 against 47.4, at 20 tokens 53.8 and
-//    53.5).
+//    while that gives two tiles a compute unit and, for 8-bit codes, most experts
+//    have a route, else 4 (8-bit codes at 8 tokens 39.5 against 47.4, at 20
+//    tokens 53.8 and 53.5; 4-bit codes at 14 tokens 36.8 against 35.5, half 34.8
+//    and 32.7).
 //    128 rows to a = 232 wide (1700 tokens, a = 212: 138.8 against 153.3 on
 //    256x8; 2048 tokens, a = 256: 170.9 and 160.5), 480 otherwise (Granite
 //    1500 tokens, a = 300: 54.0 and 62.0; 2800, a = 560: 93.7 and 84.9): the
@@ -1238,7 +1239,7 @@ static WrTile wr_tile(int64_t n_routes, int E, int64_t cols, int kin, int mode, 
       return {128, 4, 2};
     }
     if (upto(!wide ? 56 : bits == 4 ? 44 : f16 ? 48 : 56))
-      return {64, n_routes > 2 * E && E * mtiles(64) * cols >= 2 * cus ? 8 : 4, 2};
+      return {64, (bits == 4 || n_routes > 2 * E) && E * mtiles(64) * cols >= 2 * cus ? 8 : 4, 2};
     if (mode == kGgGateUp && bits == 4 && !f16) {
       if (wide && upto(400)) return {128, 4, 4};
       // Tiles of E experts of a / 128 + 1/2 m-tiles, two a compute unit: the
