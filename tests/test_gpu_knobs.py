@@ -52,7 +52,7 @@ def test_override_gives_default_bits(default_outputs, env, tmp_path):
             np.testing.assert_array_equal(got[k], ref, err_msg=k)
     if "TFM_GGEMM_SB_LAYOUT" in env:
         assert "TFM_GGEMM_SB_LAYOUT=1 has no effect" in res.stderr
-    # A top-k kernel of its own: to 64 tokens by itself, and as the override says.
-    split = int(env.get("TFM_ROUTER_SPLIT_MAX_TOKENS", 64))
+    # A top-k kernel of its own: to 192 tokens by itself, and as the override says.
+    split = int(env.get("TFM_ROUTER_SPLIT_MAX_TOKENS", 192))
     for name, T in (("olmoe", 32), ("granite", 64), ("olmoe", 300), ("granite", 1000)):
         assert got[f"topk_{name}_{T}_4"] == (1 if T <= split else 0), (name, T)

@@ -160,10 +160,10 @@ def test_scale_alignment(gpu, dtype, bits, Kin):
         np.testing.assert_array_equal(got[shift], got[0, 0])
 
 
-# Around the router kernels' switches (64 and 1024 tokens), token counts off 4
+# Around the router kernels' switches (64, 192 and 1024 tokens), token counts off 4
 # and 16, every hidden width with a kernel, expert counts on both sides of 40
 # and 48; infinite, NaN and subnormal rows. Bit for bit.
-@pytest.mark.parametrize("T", [64, 65, 131, 1024, 1025, 1043])
+@pytest.mark.parametrize("T", [64, 65, 131, 192, 193, 1024, 1025, 1043])
 @pytest.mark.parametrize("route,H,E", [("olmoe", 2048, 64), ("granite", 1536, 40), ("olmoe", 1024, 41),
                                        ("granite", 512, 7), ("olmoe", 512, 49)])
 def test_prefill_router(gpu, route, H, E, T):
@@ -193,7 +193,7 @@ def test_prefill_router(gpu, route, H, E, T):
 
 # The same kernels on half storage, whose router is affine and dequantised first:
 # 4- and 16-token workgroups, half subnormals, infinities and NaN.
-@pytest.mark.parametrize("T", [65, 1024, 1025, 1043])
+@pytest.mark.parametrize("T", [193, 1024, 1025, 1043])
 @pytest.mark.parametrize("route,H,E,router_bits", [("olmoe", 2048, 64, 4), ("granite", 1536, 40, 4), ("olmoe", 1024, 49, 8),
                                                    ("granite", 512, 7, 8)])
 def test_prefill_router_half(gpu, route, H, E, router_bits, T):

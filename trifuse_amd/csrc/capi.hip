@@ -252,10 +252,11 @@ static bool ds_prefetch() {
 }
 
 // Tokens up to which the grouped path runs the router as a logits kernel and a
-// top-k kernel (one wave a (token, expert) pair spreads the router over the
-// chip: logits, top-k and scatter 14.3 us at 45 tokens, against 16.3 for the
-// fused router kernel and its scatter, and 5 us less a layer; at 100 tokens level,
-// at 512 22.6 and 17.2). Unset 64, and whatever the tokens at up to 256 routes,
+// top-k kernel, whose many small workgroups spread it over the chip; the fused
+// kernel takes 4 tokens a workgroup, one a compute unit. us a layer, split against
+// fused: OLMoE 97 tokens 81.2 and 83.8, 128 tokens 83.9 and 86.4, 160 tokens 88.2
+// and 88.7, 192 tokens level (Granite level from 64 to 128); logits, top-k and
+// scatter at 512 tokens 22.6 and 17.2. Unset 192, and whatever the tokens at up to 256 routes,
 // where top-k and grouping are one kernel; TFM_ROUTER_SPLIT_MAX_TOKENS sets the
 // tokens alone.
 static bool router_split(int T, int64_t R) {
@@ -270,7 +271,7 @@ static bool router_split(int T, int64_t R) {
     }
     return (int)n;
   }();
-  return v >= 0 ? T <= v : T <= 64 || R <= 256;
+  return v >= 0 ? T <= v : T <= 192 || R <= 256;
 }
 
 static bool fused_decode(const tfm_geometry& g, int64_t R) {
