@@ -2,7 +2,8 @@
 //
 // Two kernels: ggemm_wr_kernel (weights in registers; input widths a multiple
 // of 128, described below at its definition) and ggemm_kernel, for odd
-// multiples of 64:
+// multiples of 64, 8-bit codes with bf16 storage of many rows (lds_dequant) and
+// scales or biases that start off a 4-byte boundary:
 //
 // Each workgroup computes a BM x BN tile of one expert's output with eight
 // waves, two per SIMD, so that one wave's loads, dequantisation and LDS
@@ -1043,7 +1044,7 @@ __global__ __launch_bounds__(WV * 64, (wr_waves_per_simd<BM>())) void ggemm_wr_k
   // (copying S+1 into the other stage on the way), barrier. With an odd
   // count the loop runs one more super-step on zero activations. Scale chunk
   // c + 1 is requested in super-step 4c: the last read of its ring slot's
-  // old chunk c - 1 was before the barrier that ended super-step 4c - 2, and
+  // old chunk (c - 1 in a ring of two) was before the barrier that ended super-step 4c - 2, and
   // its first read comes in super-step 4c + 3.
   auto main_loop = [&](auto mbl_tag) {
     for (int kt = 0; kt < KT; kt += 2) {
@@ -1179,7 +1180,9 @@ struct WrTile {
 //    layer, gate/up and down, against the other tiles: OLMoE 400 tokens 106.8
 //    and 114.4, 512 tokens 118.5 and 125.0, 1111 tokens 193.3 and 203.7; past
 //    the fit it loses: 700 tokens 162.5 and 136.1, 900 tokens 183.9 and 170.2.
-//    Not 8-bit codes, whose raw weights leave it too few registers.
+//    Not 8-bit codes, whose raw weights leave it too few registers. (The lines
+//    are those of evenly spread routes; half storage, whose affine routers spread
+//    them more, gains earlier: 360 tokens gate/up 55.0 on 64x8 and 48.2.)
 //  * Down. 64 x 4 up to a = 44 (OLMoE 300 tokens, a = 38: 29.2 against 32.8 on
 //    128x4; 400 tokens: 34.7 and 34.2), then 128 x 4 (512 tokens 38.2 against
 //    42.0 on 64x4 and 40.0 on 128x8; Granite 1024 tokens 27.6, 28.3 on 256x8;
