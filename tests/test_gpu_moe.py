@@ -114,7 +114,7 @@ def test_granite_batch_sweep(gpu, T):
 
 
 @pytest.mark.parametrize("name", ["granite_t768", "olmoe_t1792"])
-def test_large_tiles_below_384_routes(gpu, name):
+def test_tall_tiles_below_384_routes(gpu, name):
     """Large tiles where experts average fewer than 384 routes: Granite 768
     tokens (154 per expert: 256-row gate/up tiles in one round of the compute
     units, 128-row down tiles) and OLMoE 1792 tokens (224 per expert: 128-row
